@@ -27,6 +27,7 @@ ROOT = PACKAGE.parent
 DEFAULT_ARCH = "gfx950"
 # int8: the product library (include/wq8.h); int8_test: the test-only entry points (include/wq8_test.h), kept out of it
 LIBRARIES = {"int8": ["int8/csrc/quantize.hip", "int8/csrc/gemm.hip", "int8/csrc/gemm_bf16.hip", "int8/csrc/gemm_f16.hip",
+                      "int8/csrc/gemm_mid_bf16.hip", "int8/csrc/gemm_mid_f16.hip",
                       "int8/csrc/fewtoken.hip", "int8/csrc/abi.hip"],
              "int8_test": ["int8/csrc/test_entry.hip"]}
 HIP_FLAGS = [

@@ -198,16 +198,27 @@ def rotate_groups(x, group):
 # Per mode: (long-tile variant, short-tile variant or None). The timed choice compares both, whole tiles only (split 0)
 # and with the split-K tail (split 1: the tiles of an incomplete last wave split along K), as the reference times its
 # stream-K (wgpkernels/int8/__init__.py:180-183).
-# The block mode times 10 and 15, its tiles with the single-FMA biased fold (15, the short one, is an id the reference
-# does not use); 11, the short tile in the reference's fold order, runs when asked for by id.
+# The block mode's 10 and 15 are its tiles with the single-FMA biased fold (15, the short one, is an id the reference does
+# not use); 11 is the short tile in the reference's fold order.
 TILES = {"row": (0, 6), "exact": (1, 7), "block": (10, 15), "block+g": (12, 13), "exact+g": (14, None)}
+# Per mode: the tiles for launches of about one tile per CU (ids the reference does not use). They were faster than the
+# short tiles at every shape measured (M = 48-2000, K = 1536-13824, N = 1536-13824: by 3-50%), so the timed choice compares
+# them with the long ones, and the short tiles run when asked for by id or untimed.
+MID_TILES = {"row": 16, "exact": 17, "block": 18, "block+g": 19, "exact+g": 20}
 VARIANT_MODES = {0: "row", 2: "row", 6: "row", 1: "exact", 7: "exact", 10: "block", 11: "block", 12: "block+g", 13: "block+g",
-                 14: "exact+g", 15: "block"}
+                 14: "exact+g", 15: "block", **{v: mode for mode, v in MID_TILES.items()}}
 
 
 def tile_candidates(mode):
     """(variant, split) pairs the tile choice times for `mode`: the untimed default first."""
-    return [(v, split) for v in TILES[mode] if v is not None for split in (1, 0)]
+    return [(v, split) for v in (TILES[mode][0], MID_TILES[mode]) for split in (1, 0)]
+
+
+def _timed_tiles(mode, m, n, cus):
+    """tile_candidates(), without the mid tiles where the long tiles (about 256 x 192) fill the CUs twice over: from there
+    on the long ones are faster (M = 2000, N = 13824: by 20-35% in every mode)."""
+    long_only = m * n > 2 * cus * 256 * 192
+    return [c for c in tile_candidates(mode) if not (long_only and c[0] == MID_TILES[mode])]
 
 
 def _untimed_tile(mode, m, n, k, cus):
@@ -243,7 +254,7 @@ def _tile_plan(a, a_lo, sa, b, sb, bias, y, mode, output_is_residual):
         if loud:
             print(f"[WGPKernels] Autotuning {label}...", flush=True)
         started = time.time()
-        runs = {c: (lambda c: lambda: gemm(a, a_lo, sa, b, sb, bias, y.dtype, c[1], c[0], scratch))(c) for c in tile_candidates(mode)}
+        runs = {c: (lambda c: lambda: gemm(a, a_lo, sa, b, sb, bias, y.dtype, c[1], c[0], scratch))(c) for c in _timed_tiles(mode, m, n, state.cus)}
         timings = _tuning.time_cold(library(), runs, b.device)
         choice = min(timings, key=timings.get)
         _tuning.store.put(key, list(choice))

@@ -13,7 +13,8 @@ namespace wq8 {
 // short: 64 x 128 (hi/lo 32 x 128) on 4 waves, for inputs of few tokens. Variants 10 and 15 (15: the short block
 // tile, an id the reference does not use) fold block sums with the single-FMA biased form; 11 and the weight-group
 // variants fold in the reference's order.
-enum { TILE_LONG = 0, TILE_SHORT = 1 };
+// mid: 64-256 tokens x 32-192 channels by shape (gemm_mid.h, mid_plan below), ids 16-20, which the reference does not use.
+enum { TILE_LONG = 0, TILE_SHORT = 1, TILE_MID = 2 };
 struct Variant { int mode; bool wgroup; int tile; bool biased; };
 inline bool variant_info(int v, Variant& out) {
     switch (v) {
@@ -27,6 +28,11 @@ inline bool variant_info(int v, Variant& out) {
         case 13: out = {MODE_BLOCK, true, TILE_SHORT, false}; return true;
         case 14: out = {MODE_EXACT, true, TILE_LONG, false}; return true;
         case 15: out = {MODE_BLOCK, false, TILE_SHORT, true}; return true;
+        case 16: out = {MODE_ROW, false, TILE_MID, false}; return true;
+        case 17: out = {MODE_EXACT, false, TILE_MID, false}; return true;
+        case 18: out = {MODE_BLOCK, false, TILE_MID, true}; return true;
+        case 19: out = {MODE_BLOCK, true, TILE_MID, false}; return true;
+        case 20: out = {MODE_EXACT, true, TILE_MID, false}; return true;
     }
     return false;
 }
@@ -90,6 +96,57 @@ static int launch_finish(GemmArgs& g, hipStream_t stream) {
 }
 
 inline int cus_of(const GemmArgs& g) { return g.sms > 0 ? g.sms : 256; }
+
+// ---- mid tiles (gemm_mid.h) ---------------------------------------------------------------------------------------------
+// Tile shapes of each mode, and their time per k-tile in us (all CUs busy, weights from HBM, the share of the weights'
+// arrival at the chip taken off: MID_US_PER_MB below), measured at 60, 120 and 240 channel tiles with K = 2048 and 8192.
+enum { MID_ROW, MID_BLOCK, MID_BLOCK_G, MID_EXACT, MID_EXACT_G };
+struct MidShape { int bm, bn; float us[5]; };  // 0: the mode has no tile of this shape
+constexpr MidShape MID_SHAPES[] = {
+    //          row    block  block+g exact  exact+g
+    {64, 32,  {0.12f, 0.22f, 0.32f, 0.20f, 0.33f}}, {64, 64,   {0.15f, 0.25f, 0.34f, 0.23f, 0.37f}},
+    {64, 128, {0.00f, 0.00f, 0.00f, 0.47f, 0.57f}}, {128, 64,  {0.23f, 0.33f, 0.48f, 0.44f, 0.64f}},
+    {128, 128, {0.48f, 0.54f, 0.80f, 0.77f, 1.07f}}, {128, 160, {0.59f, 0.65f, 0.99f, 0.00f, 0.00f}},
+    {128, 192, {0.62f, 0.70f, 1.10f, 0.00f, 0.00f}}, {256, 128, {0.74f, 0.90f, 0.00f, 0.00f, 0.00f}},
+};
+constexpr int MID_SHAPE_COUNT = sizeof(MID_SHAPES) / sizeof(MID_SHAPES[0]);
+constexpr float MID_US_PER_MB = 0.13f;  // unique weight bytes of a k-tile over the whole launch
+inline int mid_column(const Variant& v) {
+    return v.mode == MODE_ROW ? MID_ROW : v.mode == MODE_BLOCK ? (v.wgroup ? MID_BLOCK_G : MID_BLOCK) : (v.wgroup ? MID_EXACT_G : MID_EXACT);
+}
+// Segments have tiles of 64 x 64 and 128 x 128 only.
+constexpr bool mid_segments(int bm, int bn) { return bm == bn; }
+
+// The shape and number of K pieces of a mid launch: the least estimated time. A round of at most one workgroup per CU costs
+// its k-tiles and about 4 us of launch, first copies and epilogue; more than one piece (split only: at most 8, of 4 k-blocks
+// or more) writes and reads back a plane of partial sums each and costs a second launch.
+struct MidPlan { int shape, pieces; };
+inline MidPlan mid_plan(const GemmArgs& g, const Variant& v, int split) {
+    const int col = mid_column(v);
+    const int64_t cus = cus_of(g), words = v.mode == MODE_EXACT && !v.wgroup ? 2 : 1;
+    MidPlan best{-1, 1};
+    double best_us = 0;
+    for (int s = 0; s < MID_SHAPE_COUNT; ++s) {
+        const MidShape& shape = MID_SHAPES[s];
+        if (shape.us[col] == 0.0f || (g.seg_rows && !mid_segments(shape.bm, shape.bn))) continue;
+        const int64_t tm = (g.m + shape.bm - 1) / shape.bm, tn = (g.n + shape.bn - 1) / shape.bn;
+        for (int pieces = 1; pieces <= (split && !g.seg_rows ? 8 : 1) && (pieces == 1 || g.kblocks / pieces >= 4); ++pieces) {
+            const int64_t groups = tm * tn * pieces, rounds = (groups + cus - 1) / cus;
+            const double unique_mb = 128e-6 * shape.bn * double(groups < cus ? groups : cus) / double(tm < cus ? tm : cus);
+            double us = double(rounds) * ((g.kblocks + pieces - 1) / pieces * (shape.us[col] + MID_US_PER_MB * unique_mb) + 4.0);
+            if (pieces > 1) us += 3.5 + 8.0 * pieces * words * g.m * g.n / 9e6;
+            if (best.shape < 0 || us < best_us) {
+                best = {s, pieces};
+                best_us = us;
+            }
+        }
+    }
+    return best;
+}
+// instantiated in gemm_mid_bf16.hip and gemm_mid_f16.hip
+template <int DT> int dispatch_mid(GemmArgs& g, const Variant& v, int split, hipStream_t stream);
+extern template int dispatch_mid<DT_BF16>(GemmArgs&, const Variant&, int, hipStream_t);
+extern template int dispatch_mid<DT_F16>(GemmArgs&, const Variant&, int, hipStream_t);
 
 // short tiles: two workgroups per CU (3 stages of 24 KiB); every other tile: one
 template <int BM, int BN, int WAVES_N, int WAVES_M, int MODE, bool WG, bool BIASED, int DT, bool SUMS, bool SEG, int BK = 128, int STAGES = 3>
@@ -250,6 +307,7 @@ static int launch_tiles(GemmArgs& g, int tile, int split, hipStream_t stream) {
 template <int DT, bool SEG>
 int dispatch_gemm(GemmArgs& g, const Variant& v, int split, hipStream_t stream) {
     if (!offsets_fit(g)) return -2;
+    if (v.tile == TILE_MID) return dispatch_mid<DT>(g, v, split, stream);
     if (v.mode == MODE_ROW) return launch_tiles<MODE_ROW, false, false, DT, SEG>(g, v.tile, split, stream);
     if (v.mode == MODE_EXACT && !v.wgroup) return launch_tiles<MODE_EXACT, false, false, DT, SEG>(g, v.tile, split, stream);
     if (v.mode == MODE_BLOCK && !v.wgroup) {
@@ -263,10 +321,13 @@ int dispatch_gemm(GemmArgs& g, const Variant& v, int split, hipStream_t stream) 
     return -4;
 }
 
-// workspace bytes of the transposed block scales: [sa_t (m x kblocks)][sb_t (n x kblocks)], each 256-byte aligned
+// workspace bytes of the transposed block scales: [sa_t (m x kblocks)][sb_t (n x kblocks)], each 256-byte aligned (none
+// for the mid tiles, which read them as they are)
 inline int64_t align256(int64_t v) { return (v + 255) / 256 * 256; }
 inline void scale_workspace(int m, int n, int k, const Variant& v, int64_t& sa_bytes, int64_t& sb_bytes) {
     const int64_t kb = (k + 127) / 128;
+    sa_bytes = sb_bytes = 0;
+    if (v.tile == TILE_MID) return;
     sa_bytes = v.mode == MODE_BLOCK ? align256(int64_t(m) * kb * 4) : 0;
     sb_bytes = v.wgroup ? align256(int64_t(n) * kb * 4) : 0;
 }
@@ -276,9 +337,15 @@ inline void scale_workspace(int m, int n, int k, const Variant& v, int64_t& sa_b
 inline void split_workspace(const GemmArgs& g, const Variant& v, int split, int64_t& slot_bytes, int64_t& counter_bytes) {
     slot_bytes = counter_bytes = 0;
     if (!split) return;
+    const int words = v.mode == MODE_EXACT && !v.wgroup ? 2 : 1;
+    if (v.tile == TILE_MID) {
+        // planes of m x n words, as the deep split's
+        const int pieces = mid_plan(g, v, split).pieces;
+        if (pieces > 1) slot_bytes = align256(int64_t(pieces) * words * g.m * g.n * 4);
+        return;
+    }
     const TileShape t = tile_shape(g, v);
     const int tiles = ((g.m + t.bm - 1) / t.bm) * ((g.n + t.bn - 1) / t.bn);
-    const int words = v.mode == MODE_EXACT && !v.wgroup ? 2 : 1;
     if (const int deep = g.seg_rows ? 0 : deep_pieces(tiles, g.kblocks, cus_of(g) * t.per_cu, split)) {
         // deep split: `deep` planes (two per piece with the exact mode's hi and lo) of m x n words, no counters
         slot_bytes = align256(int64_t(deep) * words * g.m * g.n * 4);
