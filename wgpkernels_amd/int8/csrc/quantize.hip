@@ -175,9 +175,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(prep_w
 #pragma unroll
             for (int j = 0; j < 8; ++j) amax = fmaxf(amax, __builtin_fabsf(v[j]));
         }
-#pragma unroll
-        for (int d = 32; d >= 1; d >>= 1) amax = fmaxf(amax, xor_shfl(amax, d));
-        amax = block_max4(amax, lds4);
+        amax = block_max4(wave_max(amax), lds4);
         const float inv = amax > 0.0f ? 127.0f / amax : 0.0f;
         if (tid == 0) p.scale[r] = div127(amax * group_norm(group));
         for (int i = 0; i < iters; ++i) {
@@ -289,8 +287,7 @@ __global__ void __launch_bounds__(256 * G) prep_wide(PrepArgs p) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) amax = fmaxf(amax, __builtin_fabsf(v[j][e]));
     }
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) amax = fmaxf(amax, xor_shfl(amax, d));
+    amax = wave_max(amax);
     if ((tid & 63) == 0) lds[tid >> 6] = amax;
     __syncthreads();
     amax = lds[0];

@@ -143,7 +143,41 @@ WQ8_DEVICE int rne_int(float t) { return int(__builtin_rintf(t)); }
 WQ8_DEVICE int rne_low_byte(float t) { return int(__builtin_bit_cast(uint32_t, t + 0x1.8p23f)); }
 
 // ---- cross-lane -------------------------------------------------------------------------------------------
-WQ8_DEVICE float xor_shfl(float v, int mask) { return __shfl_xor(v, mask, 64); }
+// The value of lane ^ MASK, on the vector ALU (__shfl_xor goes through ds_bpermute, an LDS round trip): DPP within a row of
+// 16 lanes (quad_perm for 1-3, row_half_mirror = 7, row_ror:8 = 8; 4 and 6 as 7 ^ 3 and 7 ^ 1), v_permlane16_swap and
+// v_permlane32_swap (gfx950) across rows and halves. Every lane of the wave is active.
+template <int CTRL> WQ8_DEVICE float dpp_f(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
+}
+// v_permlane16_swap of v with itself exchanges rows 1 and 0, 3 and 2 of the two copies: .a holds the even rows' values in
+// both rows of a pair, .b the odd rows'. permlane32: the same for the halves of the wave.
+struct LanePair { float a, b; };
+WQ8_DEVICE LanePair swap16(float v) {
+    const uint32_t u = __builtin_bit_cast(uint32_t, v);
+    const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    return {__builtin_bit_cast(float, uint32_t(r[0])), __builtin_bit_cast(float, uint32_t(r[1]))};
+}
+WQ8_DEVICE LanePair swap32(float v) {
+    const uint32_t u = __builtin_bit_cast(uint32_t, v);
+    const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    return {__builtin_bit_cast(float, uint32_t(r[0])), __builtin_bit_cast(float, uint32_t(r[1]))};
+}
+template <int MASK> WQ8_DEVICE float lane_xor(float v) {
+    static_assert(MASK == 1 || MASK == 2 || MASK == 4 || MASK == 6 || MASK == 8 || MASK == 16 || MASK == 24, "lane mask");
+    if constexpr (MASK == 1) return dpp_f<0xB1>(v);                  // quad_perm [1,0,3,2]
+    else if constexpr (MASK == 2) return dpp_f<0x4E>(v);             // quad_perm [2,3,0,1]
+    else if constexpr (MASK == 4) return dpp_f<0x141>(dpp_f<0x1B>(v));  // quad_perm [3,2,1,0], row_half_mirror
+    else if constexpr (MASK == 6) return dpp_f<0x141>(dpp_f<0xB1>(v));
+    else if constexpr (MASK == 8) return dpp_f<0x128>(v);            // row_ror:8
+    else if constexpr (MASK == 24) return lane_xor<16>(dpp_f<0x128>(v));
+    else {
+        const LanePair p = swap16(v);
+        return threadIdx.x & 16 ? p.a : p.b;
+    }
+}
+// v + the value of lane ^ 16, ^ 32: the sum of a pair, in either order
+WQ8_DEVICE float add_xor16(float v) { const LanePair p = swap16(v); return p.a + p.b; }
+WQ8_DEVICE float add_xor32(float v) { const LanePair p = swap32(v); return p.a + p.b; }
 
 // Max over each row of 16 lanes with DPP (no LDS round trips): quad_perm [1,0,3,2] and [2,3,0,1] combine the lanes of a
 // quad, row_half_mirror the two quads of each half row, row_mirror the two halves. Every lane of the row ends with the
@@ -151,9 +185,6 @@ WQ8_DEVICE float xor_shfl(float v, int mask) { return __shfl_xor(v, mask, 64); }
 // The values are block maxima of |x| taken with fmaxf from +0, so never NaN and never negative: for them the unsigned
 // order of the bit patterns is the float order, and the maximum runs as v_max_u32 with the DPP operand folded in (one
 // instruction per step; a float max would add a canonicalizing v_max per step).
-template <int CTRL> WQ8_DEVICE float dpp_f(float v) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
-}
 template <int CTRL> WQ8_DEVICE uint32_t dpp_u(uint32_t v) {
     return uint32_t(__builtin_amdgcn_update_dpp(0, int(v), CTRL, 0xF, 0xF, true));
 }
@@ -168,9 +199,20 @@ WQ8_DEVICE float row16_max(float amax) {
 
 // Butterfly sum over the 64 lanes (xor 32 .. 1): every lane ends with the same value (the RMS norm's pinned tree order).
 WQ8_DEVICE float wave_sum(float v) {
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) v += xor_shfl(v, d);
-    return v;
+    v = add_xor32(v);
+    v = add_xor16(v);
+    v += lane_xor<8>(v);
+    v += lane_xor<4>(v);
+    v += lane_xor<2>(v);
+    return v + lane_xor<1>(v);
+}
+// Maximum over the 64 lanes of values that are never NaN and never negative.
+WQ8_DEVICE float wave_max(float v) {
+    v = row16_max(v);
+    LanePair p = swap16(v);
+    v = fmaxf(p.a, p.b);
+    p = swap32(v);
+    return fmaxf(p.a, p.b);
 }
 
 // ---- ConvRot rotation of one 8-element chunk -------------------------------------------------------------
@@ -179,6 +221,8 @@ WQ8_DEVICE float wave_sum(float v) {
 // d0 = j & 3, d1 = (j >> 2) | ((lane & 1) << 1), d2 = (lane >> 1) & 3, d3 = (lane >> 3) & 3.
 // Stages along d0, d1, d2, d3 (up to the group): four values (a, b, c, d) along the digit give
 // s = (a + b) + (c + d) and out[i] = s - 2 * in[3 - i]. Unnormalised (the 1/sqrt(group) goes to the scale).
+// The 60 lane exchanges of a chunk at group 256 set the time of a rotated preparation (through ds_bpermute, 4096 x 5120
+// BF16 to hi / lo codes took 37.8 us, now 29.4; to row codes 36.9, now 25.0; without a rotation 16.2 and 12.6).
 WQ8_DEVICE void rotate_chunk(float* v, int group) {
     if (group < 16) return;
 #pragma unroll
@@ -192,9 +236,9 @@ WQ8_DEVICE void rotate_chunk(float* v, int group) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const float t = v[j] + v[j + 4];
-            const float s = t + xor_shfl(t, 1);
-            out[j] = s - 2.0f * xor_shfl(v[j + 4], 1);
-            out[j + 4] = s - 2.0f * xor_shfl(v[j], 1);
+            const float s = t + lane_xor<1>(t);
+            out[j] = s - 2.0f * lane_xor<1>(v[j + 4]);
+            out[j + 4] = s - 2.0f * lane_xor<1>(v[j]);
         }
 #pragma unroll
         for (int j = 0; j < 8; ++j) v[j] = out[j];
@@ -202,17 +246,16 @@ WQ8_DEVICE void rotate_chunk(float* v, int group) {
     if (group >= 64) {
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-            const float a = v[j] + xor_shfl(v[j], 2);
-            const float s = a + xor_shfl(a, 4);
-            v[j] = s - 2.0f * xor_shfl(v[j], 6);
+            const float a = v[j] + lane_xor<2>(v[j]);
+            const float s = a + lane_xor<4>(a);
+            v[j] = s - 2.0f * lane_xor<6>(v[j]);
         }
     }
     if (group >= 256) {
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-            const float a = v[j] + xor_shfl(v[j], 8);
-            const float s = a + xor_shfl(a, 16);
-            v[j] = s - 2.0f * xor_shfl(v[j], 24);
+            const float a = v[j] + lane_xor<8>(v[j]);
+            v[j] = add_xor16(a) - 2.0f * lane_xor<24>(v[j]);
         }
     }
 }
