@@ -338,6 +338,25 @@ def gemv_lines(x, weight, scale, bias=None, residual=None, residual_scale=None, 
     return y
 
 
+# One token with an input operation: applied in the GEMV's own launch for weights of at most this many values and K at most
+# this wide, where that is faster than preparing it apart (fewtoken.hip, gemv_line_act).
+LINE_ACT_MAX_WEIGHTS, LINE_ACT_MAX_K = 5120 * 5120, 5120
+
+
+def _line_act(x, weight, scale, bias, act, act_weight, eps, residual, residual_scale, out):
+    """linear() of one token through wq8_gemv_line_act, or None where it does not apply (then transform_rows and gemv_lines
+    run, with the same bits)."""
+    n, k = weight.shape
+    if (x.shape[0] != 1 or scale.dim() != 1 or k > LINE_ACT_MAX_K or n * k > LINE_ACT_MAX_WEIGHTS or k % 16 or x.dtype == torch.float32
+            or _op_width(x, act) != k or not library().has("wq8_gemv_line_act")):
+        return None
+    _check_activation(x)
+    y = torch.empty((1, n), dtype=x.dtype, device=x.device) if out is None else out
+    _lib.call("wq8_gemv_line_act", x.data_ptr(), ACTS[act], _ptr(act_weight), eps, weight.data_ptr(), scale.data_ptr(), _ptr(bias), _ptr(residual),
+              _ptr(residual_scale), y.data_ptr(), n, k, DTYPES[x.dtype], _native.gpu(x).stream())
+    return y
+
+
 # ---- prepared activations (reference: wgpkernels/int8/__init__.py:367-430) ----------------------------------------------
 class Prepared:
     """An activation prepared for one path: unquantized (transformed, rotated) rows for 'lines' / 'small', INT8 rows and
@@ -430,6 +449,10 @@ def _gemm_linear(path, x, weight, scale, bias, group, act, act_weight, eps, resi
 
 def _run_path(path, x, weight, scale, bias, group, act=None, act_weight=None, eps=0.0, residual=None, residual_scale=None, out=None):
     if path in ("lines", "small"):
+        if act and path == "lines" and not group:
+            y = _line_act(x, weight, scale, bias, act, act_weight, eps, residual, residual_scale, out)
+            if y is not None:
+                return y
         return linear_prepared(prepare(x, group, path, act, act_weight, eps), weight, scale, bias, residual, residual_scale, out)
     return _gemm_linear(path, x, weight, scale, bias, group, act, act_weight, eps, residual, residual_scale, out)
 

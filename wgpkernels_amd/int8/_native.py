@@ -37,11 +37,12 @@ SIGNATURES = {
     "wq8_small": ("i", "plpppppp" "iiiii" "ppp"),
     "wq8_small_workspace": ("-", "iiii" "p"),
     "wq8_gemv_lines": ("i", "plpppppp" "iiii" "p"),
+    "wq8_gemv_line_act": ("i", "pipf" "pppppp" "iii" "p"),
     "wq8_l2_flush": ("i", "il" "p"),
     "wq8_l2_flush_release": ("-", ""),
 }
 # entry points an older or foreign build may lack: bound when present (segments_supported() reports the first)
-OPTIONAL = {"wq8_gemm_segments", "wq8_gemm_noalloc", "wq8_quantize_at", "wq8_quantize_blocks_at", "wq8_gemm_at"}
+OPTIONAL = {"wq8_gemm_segments", "wq8_gemm_noalloc", "wq8_quantize_at", "wq8_quantize_blocks_at", "wq8_gemm_at", "wq8_gemv_line_act"}
 # the test library's entry points (include/wq8_test.h; libwgp_int8_test.so, not part of the product library)
 TEST_SIGNATURES = {
     "wq8_debug_block_sums": ("i", "ppp" "iii" "i" "p"),

@@ -287,6 +287,144 @@ template <int DT, int MT, int NIT = 1> static int dispatch_linesx(FewArgs& p, in
     }
 }
 
+// One token with its input operation applied here (RMSNorm, SwiGLU, GELU): gemv_linesx with 16 waves a workgroup, each
+// workgroup computing op(x), rounded to x's dtype as transform_rows does (the same bits, RMSNorm's tree included), straight
+// into the staged lines. x is loaded before the weights, so that the operation runs while the weights are on their way; a
+// launch and a round trip of op(x) through memory less than preparing it apart. 16 waves share one op(x), or the
+// operation (K evaluations a workgroup, 26 FP32 ops each for a gelu) would outweigh the stream.
+// For small weights only (the Python layer's LINE_ACT_MAX_*): BF16, weights from HBM, transform_rows + gemv_linesx -> this,
+// RMSNorm / gelu, us: 1536 x 1536 5.2 / 5.0 -> 4.1 / 3.6; 5120 x 5120 9.6 / 8.8 -> 9.4 / 8.7; but K = 5120, N = 13824 16.1 /
+// 15.4 -> 18.8 / 16.9 (gemv_linesx streams best in workgroups of 4 waves) and K = 8208, N = 2000 8.5 / 7.4 -> 9.9 / 8.0 (few
+// workgroups, two chunks a thread). Called one by one, the host's launch less is worth more than any of these.
+constexpr int LINE_ACT_WAVES = 16;
+template <int DT, int CH, int NIT>
+__global__ void __launch_bounds__(64 * LINE_ACT_WAVES) gemv_line_act(FewArgs p, int act, const void* act_weight, float eps) {
+    using raw = typename Elem<DT>::raw;
+    constexpr int THREADS = 64 * LINE_ACT_WAVES, CPT = (NIT * 128 + THREADS - 1) / THREADS;  // 8-element chunks a thread
+    __shared__ __attribute__((aligned(1024))) uint8_t xs[NIT * 2048];
+    __shared__ float red[LINE_ACT_WAVES], chain[256];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ch0 = (blockIdx.x * LINE_ACT_WAVES + wave) * CH;
+    const int k = p.k, n = p.n, chunks = k >> 3;
+    const raw* x = static_cast<const raw*>(p.x);
+    const raw* aw = act == ACT_RMS ? static_cast<const raw*>(act_weight) : nullptr;
+    // raw chunks of x, SwiGLU's value half or RMSNorm's weight, then the weights
+    u32x4 xr[CPT], ur[CPT];
+#pragma unroll
+    for (int j = 0; j < CPT; ++j) {
+        const int c = tid + THREADS * j;
+        xr[j] = ur[j] = u32x4{0, 0, 0, 0};
+        if (c < chunks) {
+            xr[j] = *reinterpret_cast<const u32x4*>(x + 8 * c);
+            if (act == ACT_SWIGLU) ur[j] = *reinterpret_cast<const u32x4*>(x + k + 8 * c);
+            else if (aw) ur[j] = *reinterpret_cast<const u32x4*>(aw + 8 * c);
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    const int8_t* wrow[CH];
+#pragma unroll
+    for (int c = 0; c < CH; ++c) wrow[c] = p.w + int64_t(ch0 + c < n ? ch0 + c : n - 1) * k;
+    u32x4 wv[NIT][CH];
+#pragma unroll
+    for (int it = 0; it < NIT; ++it) {
+        const int kk = it * 1024 + lane * 16, kc = kk < k ? kk : 0;
+#pragma unroll
+        for (int c = 0; c < CH; ++c) wv[it][c] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wrow[c] + kc));
+    }
+    __builtin_amdgcn_sched_barrier(0);  // every load is in flight before the operation
+    auto element = [](const u32x4& q, int e) { return Elem<DT>::to_f(raw(e & 1 ? q[e >> 1] >> 16 : q[e >> 1] & 0xffffu)); };
+    float inv = 1.0f;
+    if (act == ACT_RMS) {
+        // transform_rows's tree: slot s sums the squares of chunks s, s + 256, ... in order, the chains handed from one
+        // group of 256 threads to the next; a butterfly over each 64 slots, then ((w0 + w1) + w2) + w3
+        const int slot = tid & 255, q = tid >> 8;
+        if (q == 0) chain[slot] = 0.0f;
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < CPT; ++j)
+#pragma unroll
+            for (int g = 0; g < THREADS / 256; ++g) {
+                if (q == g) {
+                    float ss = chain[slot];
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        const float v = element(xr[j], e);
+                        ss = __builtin_fmaf(v, v, ss);
+                    }
+                    chain[slot] = ss;
+                }
+                __syncthreads();
+            }
+        const float w = wave_sum(chain[slot]);
+        if (lane == 0) red[wave] = w;
+        __syncthreads();
+        inv = rms_inverse(((red[0] + red[1]) + red[2]) + red[3], k, eps);
+    }
+#pragma unroll
+    for (int j = 0; j < CPT; ++j) {
+        const int c = tid + THREADS * j;
+        if (c < NIT * 128) {
+            u32x4 o = {0, 0, 0, 0};
+            if (c < chunks) {
+                float v[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    v[e] = element(xr[j], e);
+                    if (act == ACT_RMS) v[e] = v[e] * inv * (aw ? element(ur[j], e) : 1.0f);
+                    else if (act == ACT_SWIGLU) v[e] = wq_swiglu(v[e], element(ur[j], e));
+                    else v[e] = wq_gelu(v[e]);
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[e] = uint32_t(Elem<DT>::from_f(v[2 * e])) | uint32_t(Elem<DT>::from_f(v[2 * e + 1])) << 16;
+            }
+            // half c % 2 of line c / 128, at 16 ((c % 128) / 2)
+            *reinterpret_cast<u32x4*>(xs + (c >> 7) * 2048 + (c & 1) * 1024 + ((c & 127) >> 1) * 16) = o;
+        }
+    }
+    __syncthreads();
+    float acc[CH][2];
+#pragma unroll
+    for (int c = 0; c < CH; ++c) acc[c][0] = acc[c][1] = 0.0f;
+#pragma unroll
+    for (int it = 0; it < NIT; ++it) {
+        const bool valid = it * 1024 + lane * 16 < k;
+        u32x4 xv[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) xv[h] = *reinterpret_cast<const u32x4*>(xs + (it * 2 + h) * 1024 + lane * 16);
+#pragma unroll
+        for (int c = 0; c < CH; ++c)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                uint32_t p01, p23;
+                weight_pairs<DT>(valid ? wv[it][c][q] : 0u, p01, p23);
+                acc[c][0] = Dot2<DT>::dot(p01, xv[q >> 1][2 * (q & 1)], acc[c][0]);
+                acc[c][1] = Dot2<DT>::dot(p23, xv[q >> 1][2 * (q & 1) + 1], acc[c][1]);
+            }
+    }
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+        const float s = wave_sum(acc[c][0] + acc[c][1]);
+        if (lane == 0 && ch0 + c < n) store_out<DT>(p, 0, ch0 + c, s);
+    }
+}
+
+template <int DT, int NIT = 1> static int launch_line_act(FewArgs& p, int nit, int act, const void* act_weight, float eps, hipStream_t stream) {
+    if constexpr (NIT > 16) {
+        return -2;
+    } else {
+        if (nit != NIT) return launch_line_act<DT, NIT + 1>(p, nit, act, act_weight, eps, stream);
+        // rows per wave as gemv_linesx
+        constexpr int CH2 = NIT <= 8 ? 2 : 1;
+        if (p.n >= 8192 && CH2 == 2) {
+            const int groups = (p.n + CH2 - 1) / CH2;
+            gemv_line_act<DT, CH2, NIT><<<(groups + LINE_ACT_WAVES - 1) / LINE_ACT_WAVES, 64 * LINE_ACT_WAVES, 0, stream>>>(p, act, act_weight, eps);
+        } else {
+            gemv_line_act<DT, 1, NIT><<<(p.n + LINE_ACT_WAVES - 1) / LINE_ACT_WAVES, 64 * LINE_ACT_WAVES, 0, stream>>>(p, act, act_weight, eps);
+        }
+        return int(hipGetLastError());
+    }
+}
+
 // quads: 3-4 tokens on matrix cores. v_mfma_f32_4x4x4_{bf16,f16} computes 16 independent 4 x 4 products over 4 k each.
 // A wave takes a quad of 4 weight rows; its 16-byte load puts row i, k = k0 + 16 b .. k0 + 16 b + 15 in lane 4 b + i (4
 // rows x 256 contiguous bytes per load), whose 4 words become the A operands of 4 products (exact INT8 -> 16-bit
@@ -857,5 +995,17 @@ WQ8_API int wq8_gemv_lines(const void* x, int64_t ldx, const int8_t* w, const fl
     FewArgs p{x, ldx, w, sw, bias, residual, rscale, y, m, n, k, nullptr, nullptr, 0};
     if (dtype == DT_F16) return launch_lines<DT_F16>(p, stream);
     if (dtype == DT_BF16) return launch_lines<DT_BF16>(p, stream);
+    return -1;
+}
+
+// One token, its input operation fused (gemv_line_act): 16-bit x of 16-byte aligned rows, K % 16 == 0, K <= 16384.
+WQ8_API int wq8_gemv_line_act(const void* x, int act, const void* act_weight, float eps, const int8_t* w, const float* sw, const void* bias,
+                              const void* residual, const void* rscale, void* y, int n, int k, int dtype, hipStream_t stream) {
+    if (!n) return 0;
+    if (act < ACT_RMS || act > ACT_GELU) return -1;
+    if (n < 0 || k <= 0 || k % 16 || k > 16384 || (reinterpret_cast<uintptr_t>(x) & 15)) return -2;
+    FewArgs p{x, k, w, sw, bias, residual, rscale, y, 1, n, k, nullptr, nullptr, 0};
+    if (dtype == DT_F16) return launch_line_act<DT_F16>(p, (k + 1023) / 1024, act, act_weight, eps, stream);
+    if (dtype == DT_BF16) return launch_line_act<DT_BF16>(p, (k + 1023) / 1024, act, act_weight, eps, stream);
     return -1;
 }
