@@ -150,8 +150,8 @@ def quantize_blocks(x, group=0, act=None, act_weight=None, eps=0.0):
     lib = library()
     _check_activation(x)
     m, k = x.shape[0], _op_width(x, act)
-    q = torch.empty((m, k), dtype=torch.int8, device=x.device)
-    scale = torch.empty((m, (k + 127) // 128), dtype=torch.float32, device=x.device)
+    q = x.new_empty((m, k), dtype=torch.int8)
+    scale = x.new_empty((m, (k + 127) // 128), dtype=torch.float32)
     # RMSNorm over rows longer than the kernel keeps in registers computes the row norms first
     inv_rms = torch.empty(m, dtype=torch.float32, device=x.device) if act == "rms_norm" and k > 16384 else None
     lib.call("wq8_quantize_blocks", x.data_ptr(), q.data_ptr(), scale.data_ptr(), m, k, _row_pitch(x), DTYPES[x.dtype], group, ACTS[act],
@@ -164,9 +164,9 @@ def quantize(x, group=0, hilo=False, act=None, act_weight=None, eps=0.0):
     lib = library()
     _check_activation(x)
     m, k = x.shape[0], _op_width(x, act)
-    hi = torch.empty((m, k), dtype=torch.int8, device=x.device)
+    hi = x.new_empty((m, k), dtype=torch.int8)
     lo = torch.empty_like(hi) if hilo else None
-    scale = torch.empty(m, dtype=torch.float32, device=x.device)
+    scale = x.new_empty(m, dtype=torch.float32)
     lib.call("wq8_quantize", x.data_ptr(), hi.data_ptr(), _ptr(lo), scale.data_ptr(), m, k, _row_pitch(x), DTYPES[x.dtype], group, ACTS[act],
              _ptr(act_weight), eps, _native.gpu(x).stream())
     return hi, lo, scale
@@ -177,7 +177,7 @@ def transform_rows(x, group=0, act=None, act_weight=None, eps=0.0):
     lib = library()
     _check_activation(x)
     m, k = x.shape[0], _op_width(x, act)
-    out = torch.empty((m, k), dtype=x.dtype, device=x.device)
+    out = x.new_empty((m, k))
     lib.call("wq8_transform_rows", x.data_ptr(), out.data_ptr(), m, k, _row_pitch(x), DTYPES[x.dtype], group, ACTS[act], _ptr(act_weight), eps,
              _native.gpu(x).stream())
     return out
@@ -187,7 +187,7 @@ def rotate_groups(x, group):
     """ConvRot rotation (groups of 16, 64 or 256), rounded once to the input dtype."""
     lib = library()
     _check_activation(x)
-    out = torch.empty(x.shape, dtype=x.dtype, device=x.device)
+    out = x.new_empty(x.shape)
     lib.call("wq8_rotate_groups", x.data_ptr(), out.data_ptr(), x.shape[0], x.shape[1], _row_pitch(x), DTYPES[x.dtype], group,
              _native.gpu(x).stream())
     return out
@@ -285,7 +285,7 @@ def gemm(a, a_lo, sa, b, sb, bias, out_dtype, split=None, variant=None, out=None
     lib = library()
     m, k = a.shape
     n = b.shape[0]
-    y = torch.empty((m, n), dtype=out_dtype, device=a.device) if out is None else out
+    y = a.new_empty((m, n), dtype=out_dtype) if out is None else out
     forced = variant is not None
     if forced and variant not in VARIANT_MODES:
         raise ValueError(f"unknown INT8 GEMM variant {variant}")
@@ -318,7 +318,7 @@ def small(x, weight, scale, bias=None, residual=None, residual_scale=None, out=N
     m, k = x.shape
     n = weight.shape[0]
     state = _native.gpu(x)
-    y = torch.empty((m, n), dtype=x.dtype, device=x.device) if out is None else out
+    y = x.new_empty((m, n)) if out is None else out
     lib.wq8_small_workspace(m, n, k, state.cus, _sizes)
     stream = state.stream()
     slots, counters = _workspace(x.device, _sizes[0], _sizes[1], stream)
@@ -332,7 +332,7 @@ def gemv_lines(x, weight, scale, bias=None, residual=None, residual_scale=None, 
     lib = _lib if _lib is not None else load_library()
     _check_activation(x, aligned=False)
     m, k = x.shape
-    y = torch.empty((m, weight.shape[0]), dtype=x.dtype, device=x.device) if out is None else out
+    y = x.new_empty((m, weight.shape[0])) if out is None else out
     lib.call("wq8_gemv_lines", x.data_ptr(), _row_pitch(x), weight.data_ptr(), scale.data_ptr(), _ptr(bias), _ptr(residual),
              _ptr(residual_scale), y.data_ptr(), m, weight.shape[0], k, DTYPES[x.dtype], _native.gpu(x).stream())
     return y
@@ -351,7 +351,7 @@ def _line_act(x, weight, scale, bias, act, act_weight, eps, residual, residual_s
             or _op_width(x, act) != k or not library().has("wq8_gemv_line_act")):
         return None
     _check_activation(x)
-    y = torch.empty((1, n), dtype=x.dtype, device=x.device) if out is None else out
+    y = x.new_empty((1, n)) if out is None else out
     _lib.call("wq8_gemv_line_act", x.data_ptr(), ACTS[act], _ptr(act_weight), eps, weight.data_ptr(), scale.data_ptr(), _ptr(bias), _ptr(residual),
               _ptr(residual_scale), y.data_ptr(), n, k, DTYPES[x.dtype], _native.gpu(x).stream())
     return y
@@ -438,8 +438,12 @@ def chunk_rows(mode, k):
 
 def _gemm_linear(path, x, weight, scale, bias, group, act, act_weight, eps, residual, residual_scale, out):
     m = x.shape[0]
-    y = torch.empty((m, weight.shape[0]), dtype=x.dtype, device=x.device) if out is None else out
+    y = x.new_empty((m, weight.shape[0])) if out is None else out
     step = chunk_rows(path, weight.shape[1])
+    if m <= step:  # one chunk: no row views (about a microsecond of host time each)
+        if m:
+            linear_prepared(prepare(x, group, path, act, act_weight, eps), weight, scale, bias, residual, residual_scale, y)
+        return y
     for start in range(0, m, step):
         stop = min(m, start + step)
         prepared = prepare(x[start:stop], group, path, act, act_weight, eps)
