@@ -3,7 +3,7 @@
 //                       (one 1 KiB line per row and load instruction), exact INT8 -> BF16 / FP16 weight pairs,
 //                       v_dot2c_f32 products into FP32 accumulators, wave64 butterfly reduction. With K <= 16 KiB every
 //                       load of a wave is issued before its first product and the activations are staged in LDS per
-//                       workgroup (gemv_linesx); 3-4 tokens with K % 16 == 0 take the products on matrix cores instead
+//                       workgroup (gemv_linesx); 3-4 tokens take the products on matrix cores instead
 //                       (gemv_quads, v_mfma_f32_4x4x4, persistent workgroups); otherwise a looped kernel (gemv_lines).
 //   small (<= 32)       matrix cores: weights and activations DMA'd to LDS, INT8 weights converted exactly to BF16 /
 //                       FP16 in registers feed v_mfma_f32_16x16x32_{bf16,f16} (16 channels x 16 tokens x 32 k).
@@ -176,7 +176,7 @@ __global__ void __launch_bounds__(256) gemv_lines(FewArgs p) {
         }
 }
 
-// 1-4 tokens, 16-bit activations, K <= 16 KiB with MT * NIT <= LINEX_LINES: a wave takes CH weight rows and issues
+// 1-2 tokens, 16-bit activations, K <= 16 KiB with MT * NIT <= LINEX_LINES: a wave takes CH weight rows and issues
 // every load of them (NIT 1 KiB lines per row, 16-byte nontemporal loads) before its first product, so that the whole
 // weight matrix is requested from HBM at once instead of a few lines per wave and round trip; the grid's many short
 // waves keep every CU's loads in flight. Exact INT8 -> 16-bit weight pairs, v_dot2c products, wave64 butterfly. The
@@ -269,8 +269,8 @@ __global__ void __launch_bounds__(64 * WPG) gemv_linesx(FewArgs p) {
 
 template <int DT, int CH, int NIT, int MT> static int launch_linesx(FewArgs& p, hipStream_t stream) {
     const int groups = (p.n + CH - 1) / CH;
-    // 8 waves per workgroup (the staged activations shared by twice the rows) at N < 8192 for 2-4 tokens, and for one
-    // token with rows up to 8 KiB: measured 10% faster at 3-4 tokens, K = N = 5120, 9% at 2 tokens, K = 13824, N = 5120
+    // 8 waves per workgroup (the staged activations shared by twice the rows) at N < 8192 for 2 tokens, and for one
+    // token with rows up to 8 KiB: measured 9% faster at 2 tokens, K = 13824, N = 5120
     // and 5% at one token, K = N = 5120; slower at N = 13824 and for one token at K = 13824
     if (p.n < 8192 && (MT >= 2 || NIT <= 8)) gemv_linesx<DT, CH, NIT, MT, 8><<<(groups + 7) / 8, 512, 0, stream>>>(p);
     else gemv_linesx<DT, CH, NIT, MT><<<(groups + 3) / 4, 256, 0, stream>>>(p);
@@ -445,7 +445,9 @@ template <> struct Mfma4<DT_F16> {
     static WQ8_DEVICE v4f run(op a, op b, v4f c) { return __builtin_amdgcn_mfma_f32_4x4x4f16(a, b, c, 0, 0, 0); }
 };
 
-template <int DT, int NL, int CG, int S>
+// TAIL: K % 16 != 0. The chunks hold K rounded down to 16; the 1-3 words of each row left over are one more product of the
+// waves of range 0 (block b takes word b, blocks past them zeros), their activations staged beside the chunks.
+template <int DT, int NL, int CG, int S, bool TAIL>
 __global__ void __launch_bounds__(64 * CG * S) gemv_quads(FewArgs p, int groups) {
     using op = typename Mfma4<DT>::op;
     constexpr int W = CG * S;
@@ -454,17 +456,26 @@ __global__ void __launch_bounds__(64 * CG * S) gemv_quads(FewArgs p, int groups)
     constexpr uint32_t OUT_OF_RANGE = 0x80000000u;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int cg = wave % CG, s = wave / CG;
-    const int k = p.k, n = p.n;
+    const int k_row = p.k, k = TAIL ? k_row & ~15 : k_row, n = p.n;  // row length, and the part of it in whole chunks of 16
     const int b = lane >> 2, q4 = lane & 3;
     const sgpr4 rx = buffer_rsrc(p.x, x_span_bytes(p));
+    __shared__ __attribute__((aligned(16))) uint32_t xt[TAIL ? 128 : 4];  // pairs 2 h, 2 h + 1 of lane's word: xt[64 h + lane]
+    const bool tail_lane = TAIL && 4 * b < k_row - k;
+    if constexpr (TAIL) {
+        if (wave < 2)
+            bdma4(rx, tail_lane && q4 < p.m ? (uint32_t(q4) * uint32_t(p.ldx) + uint32_t(k + 4 * b + 2 * wave)) * 2u : OUT_OF_RANGE, xt + 64 * wave);
+    }
 #pragma unroll
     for (int q = wave; q < S * NL * 2; q += W) {
         const int kk = (q >> 1) * 256 + 16 * b + 8 * (q & 1);
         bdma16(rx, q4 < p.m && kk < k ? (uint32_t(q4) * uint32_t(p.ldx) + uint32_t(kk)) * 2u : OUT_OF_RANGE, xs + q * 1024);
     }
-    auto issue = [&](int g, u32x4 (&wv)[NL]) {
+    auto issue = [&](int g, u32x4 (&wv)[NL], uint32_t& wt) {
         const int row = (g * CG + cg) * 4 + q4;
-        const int8_t* wrow = p.w + int64_t(row < n ? row : n - 1) * k;
+        const int8_t* wrow = p.w + int64_t(row < n ? row : n - 1) * k_row;
+        if constexpr (TAIL) {
+            if (s == 0) wt = tail_lane ? *reinterpret_cast<const uint32_t*>(wrow + k + 4 * b) : 0u;
+        }
 #pragma unroll
         for (int l = 0; l < NL; ++l) {
             const int kk = (s * NL + l) * 256 + 16 * b;  // past K: any row bytes, against zero activations
@@ -472,7 +483,7 @@ __global__ void __launch_bounds__(64 * CG * S) gemv_quads(FewArgs p, int groups)
         }
     };
     // products of one group, block partials -> LDS slot, barrier, one thread per (row, token) adds and stores
-    auto finish = [&](int g, int slot, const u32x4 (&wv)[NL]) {
+    auto finish = [&](int g, int slot, const u32x4 (&wv)[NL], uint32_t wt) {
         v4f acc[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) acc[q] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
@@ -487,6 +498,13 @@ __global__ void __launch_bounds__(64 * CG * S) gemv_quads(FewArgs p, int groups)
                 weight_pairs<DT>(wv[l][q], p01, p23);
                 const u32x4& xh = q < 2 ? x0 : x1;
                 acc[q] = Mfma4<DT>::run(__builtin_bit_cast(op, u32x2{p01, p23}), __builtin_bit_cast(op, u32x2{xh[2 * (q & 1)], xh[2 * (q & 1) + 1]}), acc[q]);
+            }
+        }
+        if constexpr (TAIL) {
+            if (s == 0) {
+                uint32_t p01, p23;
+                weight_pairs<DT>(wt, p01, p23);
+                acc[0] = Mfma4<DT>::run(__builtin_bit_cast(op, u32x2{p01, p23}), __builtin_bit_cast(op, u32x2{xt[lane], xt[64 + lane]}), acc[0]);
             }
         }
         float v[4];
@@ -512,30 +530,31 @@ __global__ void __launch_bounds__(64 * CG * S) gemv_quads(FewArgs p, int groups)
         }
     };
     u32x4 wa[NL], wb[NL];
+    uint32_t ta = 0, tb = 0;
     const int G = gridDim.x;
     int g = blockIdx.x;
-    issue(g, wa);
+    issue(g, wa, ta);
     bool first = true;
     for (;;) {
         // even step: products of wa while wb's loads fly
         if (g + G < groups) {
-            issue(g + G, wb);
+            issue(g + G, wb, tb);
             wait_vmcnt<NL>();
         } else {
             wait_vmcnt<0>();
         }
         if (first) __syncthreads();  // the staged activations of every wave have landed
         first = false;
-        finish(g, 0, wa);
+        finish(g, 0, wa, ta);
         g += G;
         if (g >= groups) break;
         if (g + G < groups) {
-            issue(g + G, wa);
+            issue(g + G, wa, ta);
             wait_vmcnt<NL>();
         } else {
             wait_vmcnt<0>();
         }
-        finish(g, 1, wb);
+        finish(g, 1, wb, tb);
         g += G;
         if (g >= groups) break;
     }
@@ -553,21 +572,24 @@ static int cu_count() {
     return cached[dev];
 }
 // grid: as many workgroups as the CUs hold at once (at most 2 per CU, measured best), never more than the groups
+template <int DT, int CG, int S, int NL, bool TAIL> static int launch_quads_nl(FewArgs& p, hipStream_t stream) {
+    static int per_cu = 0;
+    if (!per_cu) {
+        int v = 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&v, gemv_quads<DT, NL, CG, S, TAIL>, 64 * CG * S, 0) != hipSuccess || v < 1) v = 1;
+        per_cu = v < 2 ? v : 2;
+    }
+    const int groups = ((p.n + 3) / 4 + CG - 1) / CG;
+    const int grid = std::min(groups, cu_count() * per_cu);
+    gemv_quads<DT, NL, CG, S, TAIL><<<grid, 64 * CG * S, 0, stream>>>(p, groups);
+    return int(hipGetLastError());
+}
 template <int DT, int CG, int S, int NL = 1> static int launch_quads(FewArgs& p, int nl, hipStream_t stream) {
     if constexpr (NL > 8) {
         return -2;
     } else {
         if (nl != NL) return launch_quads<DT, CG, S, NL + 1>(p, nl, stream);
-        static int per_cu = 0;
-        if (!per_cu) {
-            int v = 0;
-            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&v, gemv_quads<DT, NL, CG, S>, 64 * CG * S, 0) != hipSuccess || v < 1) v = 1;
-            per_cu = v < 2 ? v : 2;
-        }
-        const int groups = ((p.n + 3) / 4 + CG - 1) / CG;
-        const int grid = std::min(groups, cu_count() * per_cu);
-        gemv_quads<DT, NL, CG, S><<<grid, 64 * CG * S, 0, stream>>>(p, groups);
-        return int(hipGetLastError());
+        return p.k % 16 ? launch_quads_nl<DT, CG, S, NL, true>(p, stream) : launch_quads_nl<DT, CG, S, NL, false>(p, stream);
     }
 }
 
@@ -578,14 +600,15 @@ static int launch_lines(FewArgs& p, hipStream_t stream) {
         // activations staged in LDS (32-bit activation offsets)
         if (nit >= 1 && nit <= 16 && x_span_fits(p)) {
             if (p.m == 1) return dispatch_linesx<DT, 1>(p, nit, stream);
-            // 3-4 tokens on matrix cores: 2 row quads x 4 k ranges per workgroup up to 8 KiB rows, 1 x 8 beyond
-            if (p.m >= 3 && p.k % 16 == 0) {
-                const int chunks = (p.k + 255) / 256;
+            // 3-4 tokens on matrix cores: 2 row quads x 4 k ranges per workgroup up to 8 KiB rows, 1 x 8 beyond. With K % 16
+            // != 0 (TAIL) too: M = 3, BF16, against the v_dot2c products K = 5124, N = 4999 12.1 -> 9.7 us, K = 1540, N = 1536
+            // 5.3 -> 3.6; against the looped kernel K = 13828, N = 5120 53.1 -> 20.4
+            if (p.m >= 3) {
+                const int chunks = ((p.k & ~15) + 255) / 256;
                 if (chunks <= 32) return launch_quads<DT, 2, 4>(p, (chunks + 3) / 4, stream);
                 return launch_quads<DT, 1, 8>(p, (chunks + 7) / 8, stream);
             }
-            if (p.m == 2) return dispatch_linesx<DT, 2>(p, nit, stream);
-            if (p.m <= 4 && nit <= LINEX_LINES / 4) return dispatch_linesx<DT, 4>(p, nit, stream);
+            return dispatch_linesx<DT, 2>(p, nit, stream);
         }
     }
     const int groups = (p.n + LINE_CH - 1) / LINE_CH, grid = (groups + 3) / 4;
