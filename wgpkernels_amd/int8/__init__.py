@@ -21,6 +21,7 @@ Paths:
 linear() picks a path per GPU, shape and token-count bucket by timing the candidates once (see choose_path()).
 """
 import ctypes
+import functools
 import time
 from contextvars import ContextVar
 from pathlib import Path
@@ -461,13 +462,30 @@ def _run_path(path, x, weight, scale, bias, group, act=None, act_weight=None, ep
     return _gemm_linear(path, x, weight, scale, bias, group, act, act_weight, eps, residual, residual_scale, out)
 
 
+def _drawn_runs(paths, x, weight, scale, bias, group, act, act_weight, eps):
+    """(path, variant, split) -> a run of that GEMM path on that long or short tile: what the path choice is decided on
+    (_policy.decide_no_coarser)."""
+    m, k = x.shape[0], weight.shape[1]
+    suffix = "+g" if _has_weight_groups(scale) else ""
+
+    def run(path, variant, split):
+        step = chunk_rows(path, k)
+        for start in range(0, m, step):
+            p = prepare(x[start:start + step], group, path, act, act_weight, eps)
+            gemm(p.x, p.lo, p.scale, weight, scale, bias, p.dtype, split, variant)
+
+    drawn = [(p, v, split) for p in paths if p in ("exact", "block") for v in TILES[p + suffix] if v is not None for split in (1, 0)]
+    return {d: functools.partial(run, *d) for d in drawn}
+
+
 _decided_paths = {}  # (m, n, k, group, act, precise, weight groups, device index) -> path
 
 
 def choose_path(x, weight, scale, bias=None, group=0, precise=False, act=None, act_weight=None, eps=0.0):
     """The path linear() takes: the fastest full-precision path while it costs at most EXACT_TOLERANCE more than 'block'
-    (always a full-precision one with precise=True). Timed once per GPU, shape, input operation and token-count bucket on
-    this call's input, with cold caches, and cached; a fixed rule applies where nothing may be timed."""
+    (always a full-precision one with precise=True), the GEMM paths timed on the long and short tiles. Timed once per GPU, shape,
+    input operation and token-count bucket on this call's input, with cold caches, and cached; a fixed rule applies where
+    nothing may be timed."""
     m, k, n = x.shape[0], weight.shape[1], weight.shape[0]
     if m > DECIDE_MAX_ROWS and not precise:
         return "block"
@@ -491,10 +509,14 @@ def choose_path(x, weight, scale, bias=None, group=0, precise=False, act=None, a
         quiet = _tuning_quietly.set(True)
         try:
             runs = {p: (lambda p: lambda: _run_path(p, x, weight, scale, bias, group, act, act_weight, eps))(p) for p in shape.candidates()}
-            timings = _tuning.time_cold(library(), runs, x.device)
+            if len(runs) > 1:
+                runs.update(_drawn_runs(shape.candidates(), x, weight, scale, bias, group, act, act_weight, eps))
+            measured = _tuning.time_cold(library(), runs, x.device)
         finally:
             _tuning_quietly.reset(quiet)
-        path = _policy.decide(timings, precise)
+        timings = {p: measured[p] for p in shape.candidates()}
+        drawn = {p: min((u for d, u in measured.items() if isinstance(d, tuple) and d[0] == p), default=t) for p, t in timings.items()}
+        path = _policy.decide_no_coarser(timings, drawn, precise)
         _tuning.store.put(key, path)
         print(f"[WGPKernels] Selected {label}: {path} ({timings[path] * 1000:.1f} us; tuned in {time.time() - started:.2f} s).", flush=True)
     _decided_paths[memo] = path
