@@ -78,16 +78,17 @@ def decide(timings, precise):
 
 
 def decide_no_coarser(timings, drawn, precise):
-    """decide() on `drawn`, the timings with the GEMM paths on the long and short tiles, for which the line between the paths
-    was drawn. Tiles that are faster for some sizes make a call faster but never coarser: decided on the best tiles (`timings`),
-    18 of 133 shapes (M = 64-2000, K and N 1536-13824) went from 'exact' to 'block' (M = 100, K = 13824, N = 5120: exact 54.4
-    and block 50.3 us on the drawn tiles, 44.7 and 35.9 on the best) and two from 'small' to 'exact'. 'block' gives way to a
-    full-precision path whose best tile costs no more than the drawn 'block', and near the line (DRAWN_BAND) to one within
-    EXACT_TOLERANCE of it: a faster preparation takes the same time off both paths and so moves their ratio past the line
-    (M = 256, K = 13824, N = 5120: 69.5 / 64.6 us = 1.08 became 62.0 / 55.9 = 1.11).
-    'lines' and 'small' read the inputs as they are, where 'exact' makes hi/lo codes of them: it takes their place only when
-    more than EXACT_TOLERANCE faster (the two are within 3% at M = 8-32, K = 5120, N = 27648, and a faster preparation alone
-    turned them: the error of a gated feed-forward block of 13 tokens went from 2.2e-3 to 2.5e-3)."""
+    """decide() on `drawn`, the timings with the GEMM paths on the long and short tiles, for which the line between the
+    paths was drawn. Tiles that are faster for some sizes make a call faster but never coarser: decided on the best
+    tiles (`timings`), 19 of 133 shapes (M = 64-2000, K 1536-13824, N 1536-27648) went from 'exact' to 'block' (M = 100,
+    K = 13824, N = 5120: exact 54.4 and block 50.3 us on the drawn tiles, 44.7 and 35.9 on the best) and two from
+    'small' to 'exact'. 'block' gives way to a full-precision path whose best tile costs no more than the drawn 'block',
+    and near the line (DRAWN_BAND) to one within EXACT_TOLERANCE of it: a faster preparation takes the same time off
+    both paths and so moves their ratio past the line (M = 256, K = 13824, N = 5120: 69.5 / 64.6 us = 1.08 became 62.0 /
+    55.9 = 1.11). 'lines' and 'small' read the inputs as they are, where 'exact' makes hi/lo codes of them: it takes
+    their place only when more than EXACT_TOLERANCE faster (the two are within 3% at M = 8-32, K = 5120, N = 27648, and
+    a faster preparation alone turned them: the error of a gated feed-forward block of 13 tokens went from 2.2e-3 to
+    2.5e-3)."""
     path = decide(drawn, precise)
     if path == "exact":
         near = {p: t for p, t in drawn.items() if p in ("lines", "small") and t <= (1 + EXACT_TOLERANCE) * drawn["exact"]}
