@@ -231,6 +231,17 @@ def _untimed_tile(mode, m, n, k, cus):
     return (short_v if short and short_v is not None else long_v), 1
 
 
+def _choose_tile(mode, timings, m, n, k, cus):
+    """The fastest of the timed (variant, split) pairs; in the modes that fold in FP32 by _policy.decide_tile()."""
+    if mode in ("row", "exact"):  # INT32 sums: the same bits in every tile and split
+        return min(timings, key=timings.get)
+    own, mid = None, (MID_TILES[mode], 1)
+    if mode != "exact+g" and mid in timings:  # (the mid exact+g tile scales in an order of its own, split or not)
+        library().wq8_gemm_workspace(m, n, k, mid[0], cus, 1, _sizes)
+        own = mid if _sizes[0] else None  # planes of partial sums: K pieces of its own
+    return _policy.decide_tile(timings, own)
+
+
 # (mode, M, N, K, device) -> (variant, split, slot bytes, counter bytes) of decided shapes
 _plans = {}
 
@@ -257,7 +268,7 @@ def _tile_plan(a, a_lo, sa, b, sb, bias, y, mode, output_is_residual):
         started = time.time()
         runs = {c: (lambda c: lambda: gemm(a, a_lo, sa, b, sb, bias, y.dtype, c[1], c[0], scratch))(c) for c in _timed_tiles(mode, m, n, state.cus)}
         timings = _tuning.time_cold(library(), runs, b.device)
-        choice = min(timings, key=timings.get)
+        choice = _choose_tile(mode, timings, m, n, k, state.cus)
         _tuning.store.put(key, list(choice))
         decided = True
         if loud:

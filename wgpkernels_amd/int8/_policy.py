@@ -1,5 +1,5 @@
 """Which path serves a linear: the timed choice between the full-precision paths and 'block', and the fixed rule used
-where nothing may be timed (graph capture, compilation).
+where nothing may be timed (graph capture, compilation); and which of a mode's timed tiles a GEMM runs (decide_tile).
 
 The rule is the reference's (wgpkernels/int8/__init__.py:453-509): take the fastest full-precision path ('lines',
 'small', 'exact') while it costs at most EXACT_TOLERANCE more than 'block', else 'block'; precise=True never takes
@@ -14,6 +14,7 @@ from dataclasses import dataclass
 
 EXACT_TOLERANCE = 0.10
 DRAWN_BAND = 0.03  # see decide_no_coarser()
+WHOLE_MARGIN, ORDER_MARGIN = 0.02, 0.10  # see decide_tile()
 # few-token kernel limits (their C-ABI bounds) and the alignment their loads need
 LINE_MAX_ROWS, SMALL_MAX_ROWS = 4, 32
 LINE_K_MULTIPLE, SMALL_K_MULTIPLE = 4, 64
@@ -101,3 +102,19 @@ def decide_no_coarser(timings, drawn, precise):
         if full[best] <= (1 + (EXACT_TOLERANCE if near else 0)) * drawn["block"]:
             return best
     return path
+
+
+def decide_tile(timings, own_order=None):
+    """The tile of measured `timings` ((variant, split) -> ms) of a mode that folds in FP32, where the order of the sums
+    shows in the last bits: whole K (split 0, the same order in every tile) unless a split is more than WHOLE_MARGIN
+    faster, and `own_order`, a candidate in K pieces that no other one has, only when it is more than ORDER_MARGIN faster
+    than the rest. Two that measure the same then give the same bits in every process: at M = 32760, K = 13824, N = 5120
+    split 0 and 1 are 0.6-1.5% apart (1992 / 2003 us), and which one timing calls faster changes. At M = 512 there the mid
+    tile's 3 pieces are 6% faster than the long tile's 4 (59 / 63 us, not taken), at M = 256 25% (41 / 51 us, taken)."""
+    rest = {c: t for c, t in timings.items() if c != own_order}
+    best = min(rest, key=rest.get)
+    whole = {c: t for c, t in rest.items() if c[1] == 0 and t <= (1 + WHOLE_MARGIN) * rest[best]}
+    best = min(whole, key=whole.get, default=best)
+    if own_order in timings and (1 + ORDER_MARGIN) * timings[own_order] < rest[best]:
+        return own_order
+    return best
