@@ -107,8 +107,8 @@ int wq8_gemv_lines(const void* x, int64_t ldx, const int8_t* w, const float* sw,
                    void* y, int m, int n, int k, int dtype, wq8_stream_t stream);
 
 /* One token with its input operation (act 1-3) applied in the same launch: x one row of k values (2 k for SwiGLU), 16-byte
- * aligned, k a multiple of 16 up to 16384, dtype FP16 / BF16; the bits of wq8_transform_rows + wq8_gemv_lines. No
- * reference counterpart. */
+ * aligned, k a multiple of 16 up to 16384, dtype FP16 / BF16; the bits of wq8_transform_rows + wq8_gemv_lines. -2 where y
+ * overlaps x (residual may be x). No reference counterpart. */
 int wq8_gemv_line_act(const void* x, int act, const void* act_weight, float eps, const int8_t* w, const float* sw, const void* bias,
                       const void* residual, const void* rscale, void* y, int n, int k, int dtype, wq8_stream_t stream);
 

@@ -110,6 +110,11 @@ def _check_activation(x, aligned=True):
         raise ValueError(f"activations must be FP16, BF16 or FP32, not {x.dtype}")
 
 
+def _overlap(a, a_values, b, b_values):
+    """Whether the first a_values of a and the first b_values of b, read as contiguous, share memory."""
+    return (a.data_ptr() < b.data_ptr() + b_values * b.element_size()) and (b.data_ptr() < a.data_ptr() + a_values * a.element_size())
+
+
 def _row_pitch(x):
     """Elements between rows as the kernels read them. A one-row input's stride is meaningless (PyTorch reports
     (K, 1).t() as contiguous with stride (1, 1)), so its pitch is its width."""
@@ -361,6 +366,9 @@ def _line_act(x, weight, scale, bias, act, act_weight, eps, residual, residual_s
     n, k = weight.shape
     if (x.shape[0] != 1 or scale.dim() != 1 or k > LINE_ACT_MAX_K or n * k > LINE_ACT_MAX_WEIGHTS or k % 16 or x.dtype == torch.float32
             or _op_width(x, act) != k or not library().has("wq8_gemv_line_act")):
+        return None
+    # written in place of its input (a residual stream x = x + rs * linear(op(x))): every workgroup reads x while others store
+    if out is not None and _overlap(x, x.shape[1], out, n):
         return None
     _check_activation(x)
     y = x.new_empty((1, n)) if out is None else out

@@ -1021,12 +1021,15 @@ WQ8_API int wq8_gemv_lines(const void* x, int64_t ldx, const int8_t* w, const fl
     return -1;
 }
 
-// One token, its input operation fused (gemv_line_act): 16-bit x of 16-byte aligned rows, K % 16 == 0, K <= 16384.
+// One token, its input operation fused (gemv_line_act): 16-bit x of 16-byte aligned rows, K % 16 == 0, K <= 16384. Every
+// workgroup reads the whole of x, so y must not overlap it.
 WQ8_API int wq8_gemv_line_act(const void* x, int act, const void* act_weight, float eps, const int8_t* w, const float* sw, const void* bias,
                               const void* residual, const void* rscale, void* y, int n, int k, int dtype, hipStream_t stream) {
     if (!n) return 0;
     if (act < ACT_RMS || act > ACT_GELU) return -1;
     if (n < 0 || k <= 0 || k % 16 || k > 16384 || (reinterpret_cast<uintptr_t>(x) & 15)) return -2;
+    const uintptr_t x0 = reinterpret_cast<uintptr_t>(x), y0 = reinterpret_cast<uintptr_t>(y);
+    if (x0 < y0 + uintptr_t(n) * 2 && y0 < x0 + uintptr_t(k) * (act == ACT_SWIGLU ? 4 : 2)) return -2;
     FewArgs p{x, k, w, sw, bias, residual, rscale, y, 1, n, k, nullptr, nullptr, 0};
     if (dtype == DT_F16) return launch_line_act<DT_F16>(p, (k + 1023) / 1024, act, act_weight, eps, stream);
     if (dtype == DT_BF16) return launch_line_act<DT_BF16>(p, (k + 1023) / 1024, act, act_weight, eps, stream);
