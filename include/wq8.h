@@ -48,7 +48,8 @@ int wq8_quantize_blocks_at(const void* x, int8_t* q, float* scale, int m, int k,
                            const void* act_weight, float eps, float* inv_rms, const long long* counter, long long first, long long step,
                            wq8_stream_t stream);
 
-/* rotate(op(x)) rounded once to x's dtype: out (m, k). Replaces K8:1971; bound at I:76. */
+/* rotate(op(x)) rounded once to x's dtype: out (m, k), which may be x itself where its rows are k values apart (or, with
+ * one row, at the start of x), and overlaps x in no other way. Replaces K8:1971; bound at I:76. */
 int wq8_transform_rows(const void* x, void* out, int m, int k, int64_t ldx, int dtype, int group, int act, const void* act_weight,
                        float eps, wq8_stream_t stream);
 

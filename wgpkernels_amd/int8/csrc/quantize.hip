@@ -299,6 +299,14 @@ __global__ void __launch_bounds__(256 * G) prep_wide(PrepArgs p) {
     for (int j = 0; j < CPT; ++j) store_row_codes(p, r, k, slot + 256 * (q + G * j), chunks, inv, v[j]);
 }
 
+// Whether the rows or codes are written over input rows: prep_parts's parts each read the whole of a normalised row, where
+// one workgroup a row has it in registers (or reads its own chunk last) before it stores.
+template <int DT> static bool stores_over_input(const PrepArgs& p, int m) {
+    constexpr uintptr_t SIZE = sizeof(typename Elem<DT>::raw);
+    const uintptr_t x = reinterpret_cast<uintptr_t>(p.x), out = reinterpret_cast<uintptr_t>(p.out ? p.out : p.q);
+    return x < out + uintptr_t(m) * p.k * (p.out ? SIZE : 1) && out < x + (uintptr_t(m - 1) * p.ldx + p.k) * SIZE;
+}
+
 template <int DT, int MODE>
 static int launch_prep(const PrepArgs& p, int m, hipStream_t stream) {
     const int chunks = p.k / 8, parts = (chunks + 255) / 256;
@@ -318,13 +326,13 @@ static int launch_prep(const PrepArgs& p, int m, hipStream_t stream) {
                 else prep_wide<DT, 4, 2><<<m, 1024, 0, stream>>>(p);
                 return int(hipGetLastError());
             }
-        } else if (p.act == ACT_RMS ? m * parts <= 1024 : m <= 256 * (parts < 4 ? parts : 4)) {
+        } else if (p.act == ACT_RMS ? m * parts <= 1024 && !stores_over_input<DT>(p, m) : m <= 256 * (parts < 4 ? parts : 4)) {
             prep_parts<DT, MODE><<<m * parts, 256, 0, stream>>>(p, parts);
             return int(hipGetLastError());
         }
     }
-    // one row per workgroup; chunks per thread: the smallest count that covers the row (K = 5120 -> 3, 13824 -> 7), so no thread evaluates the
-    // activation on chunks past the row
+    // one row per workgroup; chunks per thread: the smallest count that covers the row (K = 5120 -> 3, 13824 -> 7), so no
+    // thread evaluates the activation on chunks past the row
     if (chunks <= 256) prep_rows<DT, MODE, 1><<<m, 256, 0, stream>>>(p);
     else if (chunks <= 512) prep_rows<DT, MODE, 2><<<m, 256, 0, stream>>>(p);
     else if (chunks <= 768) prep_rows<DT, MODE, 3><<<m, 256, 0, stream>>>(p);
