@@ -460,9 +460,10 @@ def _gemm_linear(path, x, weight, scale, bias, group, act, act_weight, eps, resi
     m = x.shape[0]
     y = x.new_empty((m, weight.shape[0])) if out is None else out
     step = chunk_rows(path, weight.shape[1])
-    if m <= step:  # one chunk: no row views (about a microsecond of host time each)
+    if m <= step:  # one chunk: no row views (about a microsecond of host time each) but of an output with more rows
         if m:
-            linear_prepared(prepare(x, group, path, act, act_weight, eps), weight, scale, bias, residual, residual_scale, y)
+            linear_prepared(prepare(x, group, path, act, act_weight, eps), weight, scale, bias, residual, residual_scale,
+                            y if y.shape[0] == m else y[:m])
         return y
     for start in range(0, m, step):
         stop = min(m, start + step)
