@@ -187,7 +187,7 @@ def test_block_channel_split_segments(wq, monkeypatch):
     import ctypes
     sizes = (ctypes.c_int64 * 2)()
     wq.library().wq8_gemm_workspace(512, 5120, 640, 10, 4, 0, sizes)
-    monkeypatch.setattr(wq, "_plans", {("block", 512, 5120, 640, 0): (10, 0, sizes[0], sizes[1])})  # the long biased tile
+    monkeypatch.setattr(wq, "_segment_plans", {("block", 512, 2560, 2, 640, 0): (10, sizes[0])})  # the long biased tile
     outs = [torch.empty(512, 2560, dtype=torch.bfloat16, device="cuda") for _ in range(2)]
     wq.linear_prepared_segments(p, ws, ss, bs, outs)
     torch.cuda.synchronize()

@@ -108,7 +108,7 @@ def test_mid_segments_equal_separate_linears(wq, monkeypatch, path, m, rows):
     scales = [((torch.rand(rows, generator=g) + 0.5) / 127).cuda() for _ in range(3)]
     biases = [torch.randn(rows, generator=g).bfloat16().cuda(), None, torch.randn(rows, generator=g).bfloat16().cuda()]
     prepared = wq.prepare(x, 0, path)
-    monkeypatch.setattr(wq, "_plans", {(path, m, 3 * rows, k, 0): (wq.MID_TILES[path], 1, 0, 0)})
+    monkeypatch.setattr(wq, "_segment_plans", {(path, m, rows, 3, k, 0): (wq.MID_TILES[path], 0)})
     outputs = [torch.empty(m, rows, dtype=torch.bfloat16, device="cuda") for _ in range(3)]
     wq.linear_prepared_segments(prepared, weights, scales, biases, outputs)
     for w, s, bias, y in zip(weights, scales, biases, outputs):

@@ -422,29 +422,74 @@ def linear_prepared(prepared, weight, scale, bias=None, residual=None, residual_
                 residual_scale=residual_scale)
 
 
+# (mode, M, rows of a weight, weights, K, device) -> (variant, workspace bytes) of decided segment launches
+_segment_plans = {}
+
+
+def _segments_plan(prepared, weights, scales, launch):
+    """The tile of a segments launch: its own launches timed (launch(variant, workspace bytes)), whole tiles only, as they
+    run. A plain GEMM of the joined shape does not stand for them: it has every mid tile and K pieces, segments have the
+    square mid tiles over whole K (us, block, 3 x 5120 channels, K = 5120, M = 333: long 51, mid 63, short 76; row, 3 x 1536,
+    K = 1536, M = 200: short 13.0, mid 14.6, long 28.6: the short tiles are candidates here)."""
+    mode, (m, k), count, rows = prepared.path, prepared.x.shape, len(weights), weights[0].shape[0]
+    state = _native.gpu(prepared.x)
+    kblocks, want = (k + 127) // 128, m * ((k + 127) // 128) if mode == "block" else m
+    if (any(tuple(w.shape) != (rows, k) for w in weights) or any(s.numel() not in (rows, rows * kblocks) for s in scales)
+            or prepared.scale.numel() != want):
+        raise ValueError("INT8 GEMM segment shapes do not match")
+    if not (prepared.x.is_contiguous() and prepared.scale.is_contiguous() and (prepared.lo is None or prepared.lo.is_contiguous())):
+        raise ValueError("INT8 GEMM operands must be contiguous")
+
+    def workspace_bytes(variant):
+        library().wq8_gemm_workspace(m, count * rows, k, variant, state.cus, 0, _sizes)
+        return _sizes[0]
+
+    key = f"{mode}+seg{count}|{_tuning.gemm_rows_bucket(m)}x{count * rows}x{k}|{state.name}"
+    variant = _tuning.store.get(key)
+    decided = variant is not None
+    if not decided and _tuning.is_capturing():
+        variant = _untimed_tile(mode, m, count * rows, k, state.cus)[0]
+    elif not decided:
+        label = f"INT8 GEMM {mode} {m}x({count}x{rows})x{k}"
+        loud = not _tuning_quietly.get()
+        if loud:
+            print(f"[WGPKernels] Autotuning {label}...", flush=True)
+        started = time.time()
+        candidates = [v for v in (*TILES[mode], MID_TILES[mode]) if v is not None]
+        timings = _tuning.time_cold(library(), {v: functools.partial(launch, v, workspace_bytes(v)) for v in candidates}, prepared.x.device)
+        variant = min(timings, key=timings.get)
+        _tuning.store.put(key, variant)
+        decided = True
+        if loud:
+            print(f"[WGPKernels] Selected {label}: tiles {variant} ({timings[variant] * 1000:.1f} us; tuned in {time.time() - started:.2f} s).",
+                  flush=True)
+    plan = (variant, workspace_bytes(variant))
+    if decided:
+        _segment_plans[(mode, m, rows, count, k, prepared.x.device.index)] = plan
+    return plan
+
+
 def linear_prepared_segments(prepared, weights, scales, biases, outputs):
     """outputs[s] = prepared @ (weights[s] * scales[s]).T + biases[s] for 1 to 4 linears in one GEMM launch ('exact',
     'block' or 'row' preparations, per-channel scales, equal row counts that are multiples of 8). The input is read once
-    for all of them; the tile is the one decided for the joined shape."""
+    for all of them; the tile is timed on these launches once per shape."""
     lib = library()
     if not segments_supported():
         raise RuntimeError("the loaded INT8 library has no wq8_gemm_segments")
     a, count, rows = prepared.x, len(weights), weights[0].shape[0]
     m, k = a.shape
-    n = count * rows
-    plan = _plans.get((prepared.path, m, n, k, a.device.index))
-    if plan is None:
-        joined = torch.cat(weights)
-        plan = _tile_plan(a, prepared.lo, prepared.scale, joined, torch.cat(scales), None, torch.empty((m, n), dtype=prepared.dtype, device=a.device),
-                          prepared.path, False)
-        del joined
-    variant, split, slot_bytes, counter_bytes = plan
     state = _native.gpu(a)
-    stream = state.stream()
-    slots, counters = _workspace(a.device, slot_bytes, counter_bytes, stream)
     table = lambda tensors: (ctypes.c_void_p * 4)(*[_ptr(t) for t in tensors])
-    lib.call("wq8_gemm_segments", a.data_ptr(), _ptr(prepared.lo), prepared.scale.data_ptr(), table(weights), table(scales), table(biases),
-             table(outputs), count, rows, m, k, DTYPES[prepared.dtype], variant, state.cus, split, _ptr(slots), counters, stream)
+    tables = table(weights), table(scales), table(biases), table(outputs)
+
+    def launch(variant, workspace_bytes):
+        stream = state.stream()
+        slots, _ = _workspace(a.device, workspace_bytes, 0, stream)
+        lib.call("wq8_gemm_segments", a.data_ptr(), _ptr(prepared.lo), prepared.scale.data_ptr(), *tables, count, rows, m, k,
+                 DTYPES[prepared.dtype], variant, state.cus, 0, _ptr(slots), None, stream)
+
+    plan = _segment_plans.get((prepared.path, m, rows, count, k, a.device.index))
+    launch(*(plan if plan is not None else _segments_plan(prepared, weights, scales, launch)))
     return outputs
 
 
