@@ -14,6 +14,7 @@ CASES = [
     ("block", True, {(10, 1): 62.2, (10, 0): 59.5, (18, 1): 58.7, (18, 0): 59.0}, (18, 0)),
     ("block", False, {(10, 1): 52.4, (10, 0): 53.7, (18, 1): 51.9, (18, 0): 52.0}, (18, 0)),       # mid, whole K either way
     ("block+g", True, {(12, 1): 77.4, (12, 0): 169.0, (19, 1): 76.7, (19, 0): 110.0}, (12, 1)),
+    ("block+g", False, {(12, 1): 131.0, (12, 0): 180.0, (19, 1): 132.0, (19, 0): 132.0}, (12, 1)),  # another tile: the fastest
     ("exact+g", True, {(14, 1): 40.3, (14, 0): 80.0, (20, 1): 39.0, (20, 0): 60.0}, (20, 1)),      # another order in any case
     ("row", True, {(0, 1): 30.0, (0, 0): 30.2, (16, 1): 29.9, (16, 0): 31.0}, (16, 1)),            # INT32 sums: the fastest
     ("exact", True, {(1, 1): 30.0, (1, 0): 30.2}, (1, 1)),

@@ -106,15 +106,15 @@ def decide_no_coarser(timings, drawn, precise):
 
 def decide_tile(timings, own_order=None):
     """The tile of measured `timings` ((variant, split) -> ms) of a mode that folds in FP32, where the order of the sums
-    shows in the last bits: whole K (split 0, the same order in every tile) unless a split is more than WHOLE_MARGIN
-    faster, and `own_order`, a candidate in K pieces that no other one has, only when it is more than ORDER_MARGIN faster
-    than the rest. Two that measure the same then give the same bits in every process: at M = 32760, K = 13824, N = 5120
-    split 0 and 1 are 0.6-1.5% apart (1992 / 2003 us), and which one timing calls faster changes. At M = 512 there the mid
-    tile's 3 pieces are 6% faster than the long tile's 4 (59 / 63 us, not taken), at M = 256 25% (41 / 51 us, taken)."""
+    shows in the last bits: the fastest, but whole K (split 0, the same order in every tile) unless the same tile's split is
+    more than WHOLE_MARGIN faster, and `own_order`, a candidate in K pieces that no other one has, only when it is more than
+    ORDER_MARGIN faster than the rest. A tile whose split gains nothing then gives the same bits in every process: at M =
+    32760, K = 13824, N = 5120 split 0 and 1 are 0.6-1.5% apart (1992 / 2003 us), and which one timing calls faster changes.
+    At M = 512 there the mid tile's 3 pieces are 6% faster than the long tile's 4 (59 / 63 us, not taken), at M = 256 25%
+    (41 / 51 us, taken)."""
     rest = {c: t for c, t in timings.items() if c != own_order}
     best = min(rest, key=rest.get)
-    whole = {c: t for c, t in rest.items() if c[1] == 0 and t <= (1 + WHOLE_MARGIN) * rest[best]}
-    best = min(whole, key=whole.get, default=best)
     if own_order in timings and (1 + ORDER_MARGIN) * timings[own_order] < rest[best]:
         return own_order
-    return best
+    whole = (best[0], 0)
+    return whole if rest.get(whole, float("inf")) <= (1 + WHOLE_MARGIN) * rest[best] else best
