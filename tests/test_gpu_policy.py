@@ -74,6 +74,34 @@ def test_choice_matches_cold_measurement(wq, oracle, fresh_store, k, n):
     assert sum(key.startswith("path|") for key in fresh_store.entries()) == 5  # one decision per token bucket
 
 
+@pytest.mark.parametrize("m,k,n", [(13, 5120, 13824), (64, 5120, 5120), (100, 13824, 5120), (256, 5120, 5120), (512, 5120, 5120)])
+def test_choice_never_coarser_than_on_the_drawn_tiles(wq, fresh_store, monkeypatch, m, k, n):
+    """The choice of choose_path() is decide_no_coarser()'s on what it timed: every path on its best tile, and every path on
+    the long and short tiles. The path taken costs (timed apart, weights cold) at most the rule's EXACT_TOLERANCE more than
+    the path that those tiles alone would give, and as much again for two timings' noise."""
+    from wgpkernels_amd.int8 import _policy, _tuning
+    timed, time_cold = [], _tuning.time_cold
+    monkeypatch.setattr(_tuning, "time_cold", lambda *args: timed.append(time_cold(*args)) or timed[-1])
+    x = torch.randn(m, k, device="cuda").bfloat16()
+    s = (torch.rand(n, device="cuda") + 0.5) / 127
+    bias = torch.randn(n, device="cuda").bfloat16()
+    copies = [torch.randint(-127, 128, (n, k), dtype=torch.int8, device="cuda") for _ in range(CACHE_BYTES // (n * k) + 2)]
+    print(f"path choice m={m} k={k} n={n}", flush=True)
+    chosen = wq.choose_path(x, copies[0], s, bias)
+    candidates = _policy.LinearShape(m, n, k).candidates()
+    best = next(t for t in timed if set(t) == set(candidates))
+    names = lambda t: {r if isinstance(r, str) else r[0]: u for r, u in t.items()}
+    drawn_tiles = timed[-1]
+    assert {r[1] for r in drawn_tiles if not isinstance(r, str)} <= {v for tiles in wq.TILES.values() for v in tiles}
+    drawn = names(drawn_tiles)
+    assert set(drawn) == set(candidates)
+    assert chosen == _policy.decide_no_coarser(best, drawn, False)
+    before = _policy.decide(drawn, False)
+    assert candidates.index(chosen) <= candidates.index(before)  # candidates() goes from fine to coarse
+    allowed = drawn[before] * (1 + _policy.EXACT_TOLERANCE) ** 2
+    assert cold_path_ms(wq, chosen, x, copies, s, bias) <= allowed, (chosen, before, best, drawn)
+
+
 def test_long_inputs_take_block_untimed(wq, fresh_store):
     x = torch.zeros(4097, 256, dtype=torch.bfloat16, device="cuda")
     w = torch.zeros(64, 256, dtype=torch.int8, device="cuda")

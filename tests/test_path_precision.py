@@ -22,6 +22,12 @@ CASES = [
     (512, dict(exact=27.0, block=24.0), dict(exact=32.7, block=26.2), False, False, "block"),       # well past it and slower
     (16, dict(exact=41.3, block=47.4), dict(exact=68.6, block=51.2), True, False, "exact"),         # finer and no slower
     (100, dict(exact=44.7), dict(exact=54.4), False, True, "exact"),
+    (13, dict(small=36.0, exact=20.0), dict(exact=33.0), False, True, "exact"),   # near on the drawn tiles, far on the best
+    (13, dict(small=36.0, exact=20.0, block=34.0), dict(exact=33.0, block=34.0), False, False, "exact"),
+    (100, dict(exact=50.0, block=25.0), dict(exact=54.0, block=50.0), False, False, "exact"),  # finer on the drawn tiles: stays
+    (333, dict(exact=50.0, block=42.0), dict(exact=56.0, block=50.0), False, False, "exact"),  # 'block' before, as fast now
+    (333, dict(exact=54.0, block=42.0), dict(exact=59.0, block=50.0), False, False, "block"),  # 18% over it, and slower
+    (100, dict(exact=44.7, block=35.5), dict(exact=47.4, block=40.9), False, False, "exact"),  # a faster preparation: 1.08 to 1.16
 ]
 
 

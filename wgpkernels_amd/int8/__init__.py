@@ -528,8 +528,10 @@ def _run_path(path, x, weight, scale, bias, group, act=None, act_weight=None, ep
 
 
 def _drawn_runs(paths, x, weight, scale, bias, group, act, act_weight, eps):
-    """(path, variant, split) -> a run of that GEMM path on that long or short tile: what the path choice is decided on
-    (_policy.decide_no_coarser)."""
+    """(path, variant, split) -> a run of each GEMM path of `paths` on the fastest of its long and short tiles: what the path
+    choice is decided on (_policy.decide_no_coarser). The tiles are timed on the bare GEMM first, as a tile choice does, so
+    that as many whole linears are timed against each other as there are paths: each more among them makes the others'
+    later launches start colder (up to 5% for a path of several launches)."""
     m, k = x.shape[0], weight.shape[1]
     suffix = "+g" if _has_weight_groups(scale) else ""
 
@@ -539,8 +541,18 @@ def _drawn_runs(paths, x, weight, scale, bias, group, act, act_weight, eps):
             p = prepare(x[start:start + step], group, path, act, act_weight, eps)
             gemm(p.x, p.lo, p.scale, weight, scale, bias, p.dtype, split, variant)
 
-    drawn = [(p, v, split) for p in paths if p in ("exact", "block") for v in TILES[p + suffix] if v is not None for split in (1, 0)]
-    return {d: functools.partial(run, *d) for d in drawn}
+    def fastest(path):
+        chunk = functools.cache(lambda: prepare(x[:chunk_rows(path, k)], group, path, act, act_weight, eps))
+        tiles = [(path, v, split) for v in TILES[path + suffix] if v is not None for split in (1, 0)]
+
+        def one(_, variant, split):
+            p = chunk()  # prepared once, by the first untimed run
+            gemm(p.x, p.lo, p.scale, weight, scale, bias, p.dtype, split, variant)
+
+        timings = _tuning.time_cold(library(), {t: functools.partial(one, *t) for t in tiles}, x.device)
+        return min(timings, key=timings.get)
+
+    return {t: functools.partial(run, *t) for t in (fastest(p) for p in paths if p in ("exact", "block"))}
 
 
 _decided_paths = {}  # (m, n, k, group, act, precise, weight groups, device index) -> path
@@ -548,9 +560,9 @@ _decided_paths = {}  # (m, n, k, group, act, precise, weight groups, device inde
 
 def choose_path(x, weight, scale, bias=None, group=0, precise=False, act=None, act_weight=None, eps=0.0):
     """The path linear() takes: the fastest full-precision path while it costs at most EXACT_TOLERANCE more than 'block'
-    (always a full-precision one with precise=True), the GEMM paths timed on the long and short tiles. Timed once per GPU, shape,
-    input operation and token-count bucket on this call's input, with cold caches, and cached; a fixed rule applies where
-    nothing may be timed."""
+    (always a full-precision one with precise=True), decided with the GEMM paths on the long and short tiles, never a coarser
+    one for a faster tile (_policy.decide_no_coarser). Timed once per GPU, shape, input operation and token-count bucket on
+    this call's input, with cold caches, and cached; a fixed rule applies where nothing may be timed."""
     m, k, n = x.shape[0], weight.shape[1], weight.shape[0]
     if m > DECIDE_MAX_ROWS and not precise:
         return "block"
@@ -574,13 +586,13 @@ def choose_path(x, weight, scale, bias=None, group=0, precise=False, act=None, a
         quiet = _tuning_quietly.set(True)
         try:
             runs = {p: (lambda p: lambda: _run_path(p, x, weight, scale, bias, group, act, act_weight, eps))(p) for p in shape.candidates()}
+            timings = drawn = _tuning.time_cold(library(), runs, x.device)
             if len(runs) > 1:
-                runs.update(_drawn_runs(shape.candidates(), x, weight, scale, bias, group, act, act_weight, eps))
-            measured = _tuning.time_cold(library(), runs, x.device)
+                few = {p: run for p, run in runs.items() if p in ("lines", "small")}
+                drawn = _tuning.time_cold(library(), {**few, **_drawn_runs(runs, x, weight, scale, bias, group, act, act_weight, eps)}, x.device)
+                drawn = {r if isinstance(r, str) else r[0]: t for r, t in drawn.items()}
         finally:
             _tuning_quietly.reset(quiet)
-        timings = {p: measured[p] for p in shape.candidates()}
-        drawn = {p: min((u for d, u in measured.items() if isinstance(d, tuple) and d[0] == p), default=t) for p, t in timings.items()}
         path = _policy.decide_no_coarser(timings, drawn, precise)
         _tuning.store.put(key, path)
         print(f"[WGPKernels] Selected {label}: {path} ({timings[path] * 1000:.1f} us; tuned in {time.time() - started:.2f} s).", flush=True)

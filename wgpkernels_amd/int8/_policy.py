@@ -4,7 +4,8 @@ where nothing may be timed (graph capture, compilation); and which of a mode's t
 The rule is the reference's (wgpkernels/int8/__init__.py:453-509): take the fastest full-precision path ('lines',
 'small', 'exact') while it costs at most EXACT_TOLERANCE more than 'block', else 'block'; precise=True never takes
 'block'; above DECIDE_MAX_ROWS tokens 'block' is taken untimed. Per-(channel, k-block) weight scales leave 'exact' as
-the only full-precision path.
+the only full-precision path. It is applied to the long and short tiles' times (decide_no_coarser): where a mid tile makes
+'block' faster than that, a full-precision path can cost more than EXACT_TOLERANCE over the 'block' it leaves.
 
 The fixed rule's thresholds are MI355X measurements, not the reference's RTX 5090 ones: with cold weights 'lines' is
 the fastest path up to 4 tokens and 'small' up to 32 at the Wan widths (K, N in {5120, 13824}), where 'exact' (two
@@ -13,7 +14,7 @@ INT8 passes plus a quantize launch) was 20-45% slower.
 from dataclasses import dataclass
 
 EXACT_TOLERANCE = 0.10
-DRAWN_BAND = 0.03  # see decide_no_coarser()
+DRAWN_BAND = 0.06  # see decide_no_coarser()
 WHOLE_MARGIN, ORDER_MARGIN = 0.02, 0.10  # see decide_tile()
 # few-token kernel limits (their C-ABI bounds) and the alignment their loads need
 LINE_MAX_ROWS, SMALL_MAX_ROWS = 4, 32
@@ -83,16 +84,20 @@ def decide_no_coarser(timings, drawn, precise):
     paths was drawn. Tiles that are faster for some sizes make a call faster but never coarser: decided on the best
     tiles (`timings`), 19 of 133 shapes (M = 64-2000, K 1536-13824, N 1536-27648) went from 'exact' to 'block' (M = 100,
     K = 13824, N = 5120: exact 54.4 and block 50.3 us on the drawn tiles, 44.7 and 35.9 on the best) and two from
-    'small' to 'exact'. 'block' gives way to a full-precision path whose best tile costs no more than the drawn 'block',
-    and near the line (DRAWN_BAND) to one within EXACT_TOLERANCE of it: a faster preparation takes the same time off
-    both paths and so moves their ratio past the line (M = 256, K = 13824, N = 5120: 69.5 / 64.6 us = 1.08 became 62.0 /
-    55.9 = 1.11). 'lines' and 'small' read the inputs as they are, where 'exact' makes hi/lo codes of them: it takes
-    their place only when more than EXACT_TOLERANCE faster (the two are within 3% at M = 8-32, K = 5120, N = 27648, and
-    a faster preparation alone turned them: the error of a gated feed-forward block of 13 tokens went from 2.2e-3 to
-    2.5e-3)."""
+    'small' to 'exact'. So the path taken may be slower than another one is now, but not than what ran on the drawn tiles:
+    - 'block' gives way to a full-precision path whose best tile costs no more than the drawn 'block'. Near the line
+      (DRAWN_BAND) one within EXACT_TOLERANCE of it will do: a faster preparation takes more of 'block' than of 'exact' and
+      so moves their ratio past the line (M = 100, K = 13824, N = 5120, gelu: 54.4 / 50.3 us = 1.08 became 47.4 / 40.9 =
+      1.16). Of 560 shapes timed three times, 11 of 1608 choices were coarser than before the faster preparations without a
+      band, 4 with 0.03, 2 with 0.06 and 0.08; what the band of 0.06 adds measured at most 1% slower than before.
+    - 'lines' and 'small' read the inputs as they are, where 'exact' makes hi/lo codes of them: it takes their place only
+      when more than EXACT_TOLERANCE faster, on the drawn or on the best tiles (the two are within 3% at M = 8-32, K = 5120,
+      N = 27648, and a faster preparation alone turned them: the error of a gated feed-forward block of 13 tokens went from
+      2.2e-3 to 2.5e-3)."""
     path = decide(drawn, precise)
     if path == "exact":
-        near = {p: t for p, t in drawn.items() if p in ("lines", "small") and t <= (1 + EXACT_TOLERANCE) * drawn["exact"]}
+        within = lambda p, times: times[p] <= (1 + EXACT_TOLERANCE) * times["exact"]
+        near = {p: t for p, t in drawn.items() if p in ("lines", "small") and within(p, drawn) and within(p, timings)}
         return min(near, key=near.get, default=path)
     if path == "block":
         full = {p: t for p, t in timings.items() if p != "block"}

@@ -23,7 +23,7 @@ import torch
 
 from . import _native
 
-TUNING_VERSION = 5  # decisions timed on other kernels or by another rule (an older version's file) do not stand
+TUNING_VERSION = 6  # decisions timed on other kernels or by another rule (an older version's file) do not stand
 DEFAULT_PATH = Path.home() / ".triton" / "autotune" / "wgpkernels_amd_int8.json"
 ROUNDS = 5
 # 4 MiB of L2 per XCD x 8 XCDs plus the 256 MiB MALL, read twice over
