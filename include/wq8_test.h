@@ -23,6 +23,9 @@ int wq8_debug_block_sums(const int8_t* a, const int8_t* b, int32_t* sums, int m,
  * in-run matrix-core ceiling. */
 int wq8_debug_mfma_probe(const void* operands, int* out, int blocks, int iters, int shape, wq8_stream_t stream);
 
+/* The tile of a mid variant (16-20): plan = {tokens, channels, K pieces}; seg_rows: rows of each segment, or 0. Host only. */
+int wq8_debug_mid_plan(int m, int n, int k, int variant, int sms, int split, int seg_rows, int* plan);
+
 #ifdef __cplusplus
 }
 #endif

@@ -57,11 +57,14 @@ def wq():
 @pytest.fixture
 def whole_tiles(wq, monkeypatch, tmp_path):
     """The tile choice timed from an empty store over whole tiles only (split 0): every tile it can pick for a mode folds
-    in the same order (block: 10 and 15 both biased; row and exact: INT32), so that outputs of different shapes, chunks
-    or entry points compare bit for bit whatever tile wins. (With split 1 the split-K order depends on the tiles.)"""
+    in the same order (block: 10, 15 and 18 all biased; row and exact: INT32), so that outputs of different shapes, chunks
+    or entry points compare bit for bit whatever tile wins. (With split 1 the split-K order depends on the tiles; the mid
+    tile of exact+g scales in an order of its own.)"""
     monkeypatch.setattr(wq._tuning, "store", wq._tuning.Store(str(tmp_path / "tiles.json")))
     monkeypatch.setattr(wq, "_plans", {})
-    monkeypatch.setattr(wq, "tile_candidates", lambda mode: [(v, 0) for v in wq.TILES[mode] if v is not None])
+    monkeypatch.setattr(wq, "_segment_plans", {})
+    tiles = lambda mode: (*wq.TILES[mode], None if mode == "exact+g" else wq.MID_TILES[mode])
+    monkeypatch.setattr(wq, "tile_candidates", lambda mode: [(v, 0) for v in tiles(mode) if v is not None])
     return wq
 
 

@@ -58,11 +58,15 @@ def test_quantize_at_entry_points(wq, oracle, act):
     np.testing.assert_array_equal(sr.cpu().numpy().view(np.uint32), sr_ref.view(np.uint32))
 
 
-@pytest.mark.parametrize("mode,variant", [("row", 0), ("row", 6), ("block", 10), ("block", 11), ("block", 15), ("exact", 1), ("exact", 7)])
-def test_gemm_at_offsets_vs_oracle(wq, oracle, mode, variant):
+@pytest.mark.parametrize("mode,variant,k,split", [("row", 0, 384, 0), ("row", 6, 384, 0), ("block", 10, 384, 0), ("block", 11, 384, 0),
+                                                   ("block", 15, 384, 0), ("exact", 1, 384, 0), ("exact", 7, 384, 0),
+                                                   ("row", 16, 384, 0), ("exact", 17, 384, 0), ("block", 18, 384, 0),
+                                                   ("row", 16, 8192, 1), ("exact", 17, 8192, 1), ("block", 18, 8192, 1)])
+def test_gemm_at_offsets_vs_oracle(wq, oracle, mode, variant, k, split):
     """wq8_gemm_at with shifted input rows (in_first + counter * in_step), shifted output / residual rows and per-span
-    residual scales; only the addressed output rows are written, and they equal the oracle bit for bit."""
-    m, n, k, spans = 72, 136, 384, 4
+    residual scales; only the addressed output rows are written, and they equal the oracle bit for bit. With split 1 the
+    mid tiles (16-18) run in K pieces that a second launch adds."""
+    m, n, spans = 72, 136, 4
     total = 5 * m
     g = torch.Generator().manual_seed(variant + 40)
     kb = (k + 127) // 128
@@ -85,17 +89,19 @@ def test_gemm_at_offsets_vs_oracle(wq, oracle, mode, variant):
     counter = torch.tensor([c], dtype=torch.int64, device="cuda")
     lib = wq.library()
     sizes = (__import__("ctypes").c_int64 * 2)()
-    lib.wq8_gemm_workspace(m, n, k, variant, 256, 0, sizes)
+    lib.wq8_gemm_workspace(m, n, k, variant, 256, split, sizes)
     ws = torch.empty(max(1, sizes[0]), dtype=torch.uint8, device="cuda")
+    pieces = sizes[0] // (4 * m * n * (2 if mode == "exact" else 1)) if split else 1
+    assert (pieces > 1) == bool(split)
     print(f"gemm_at mode={mode} variant={variant} input rows {in_rows} output rows {out_rows}", flush=True)
     rc = lib.wq8_gemm_at(a_d.data_ptr(), None if lo_d is None else lo_d.data_ptr(), sa_d.data_ptr(), b_d.data_ptr(), sb_d.data_ptr(),
-                         bias_d.data_ptr(), res_d.data_ptr(), rscale_d.data_ptr(), out.data_ptr(), m, n, k, BF16, variant, 256, 0,
+                         bias_d.data_ptr(), res_d.data_ptr(), rscale_d.data_ptr(), out.data_ptr(), m, n, k, BF16, variant, 256, split,
                          ws.data_ptr(), None, counter.data_ptr(), first, step, m, n, in_first, in_step, stream())
     assert rc == 0
     torch.cuda.synchronize()
-    oracle_mode = "block_biased" if variant in BIASED else mode
+    oracle_mode = "block_biased" if variant in (*BIASED, 18) else mode
     ref = oracle.gemm(a[in_rows].numpy(), None if a_lo is None else a_lo[in_rows].numpy(), sa[in_rows].numpy(), b.numpy(), sb.numpy(),
-                      bits(bias), BF16, oracle_mode, bits(residual[out_rows]), bits(rscale[c]))
+                      bits(bias), BF16, oracle_mode, bits(residual[out_rows]), bits(rscale[c]), pieces=pieces)
     got = out.cpu()
     np.testing.assert_array_equal(bits(got[out_rows]), ref)
     assert got[:out_rows.start].abs().sum().item() == 0 and got[out_rows.stop:].abs().sum().item() == 0

@@ -39,6 +39,17 @@ CASES = [
     (16, 3, 5, 16, 256, 1), (17, 40, 9, 128, 256, 1), (18, 1, 1, 64, 256, 1), (19, 33, 17, 144, 256, 0), (20, 2, 40, 256, 256, 1),
     (17, 70, 130, 8 * 1024, 256, 1), (18, 97, 260, 12 * 1024, 256, 1),  # 8 pieces
 ]
+# segments: (m, rows of each of three weights, k, CUs counted, side of the square tile, dtype)
+SEGMENTS = [(100, 264, 640, 256, 64, torch.bfloat16), (200, 1000, 640, 256, 64, torch.bfloat16), (130, 200, 784, 4, 128, torch.bfloat16),
+            (200, 264, 640, 4, 128, torch.float16), (150, 104, 912, 2, 128, torch.float16), (99, 136, 784, 64, 64, torch.float16)]
+
+
+def mid_plan(m, n, k, variant, cus, split, seg_rows=0):
+    """(tokens, channels, K pieces) of the tile that the library gives a mid launch (host only)."""
+    from wgpkernels_amd.int8 import _native
+    plan = (ctypes.c_int * 3)()
+    assert _native.load_test_library().wq8_debug_mid_plan(m, n, k, variant, cus, split, seg_rows, plan) == 0
+    return tuple(plan)
 
 
 def p(t):
@@ -97,23 +108,27 @@ def test_mid_tiles_match_oracle(wq, oracle, index):
 
 
 @pytest.mark.parametrize("path", ["row", "exact", "block"])
-@pytest.mark.parametrize("m,rows", [(100, 264), (200, 1000)])
-def test_mid_segments_equal_separate_linears(wq, monkeypatch, path, m, rows):
+@pytest.mark.parametrize("m,rows,k,cus,tile,dtype", SEGMENTS, ids=str)
+def test_mid_segments_equal_separate_linears(wq, monkeypatch, path, m, rows, k, cus, tile, dtype):
     """Segments on the mid tiles (64 x 64 and 128 x 128; tiles that straddle two segments): the same bits as one linear per
-    weight over whole K."""
-    k = 640
+    weight over whole K, on the mid tile of that shape and on the long tile."""
+    assert mid_plan(m, 3 * rows, k, wq.MID_TILES[path], cus, 0, rows) == (tile, tile, 1)
     g = torch.Generator().manual_seed(m)
-    x = torch.randn(m, k, generator=g).bfloat16().cuda()
+    x = torch.randn(m, k, generator=g).to(dtype).cuda()
     weights = [torch.randint(-127, 128, (rows, k), generator=g, dtype=torch.int8).cuda() for _ in range(3)]
     scales = [((torch.rand(rows, generator=g) + 0.5) / 127).cuda() for _ in range(3)]
-    biases = [torch.randn(rows, generator=g).bfloat16().cuda(), None, torch.randn(rows, generator=g).bfloat16().cuda()]
+    biases = [torch.randn(rows, generator=g).to(dtype).cuda(), None, torch.randn(rows, generator=g).to(dtype).cuda()]
     prepared = wq.prepare(x, 0, path)
+    wants = [[wq.gemm(prepared.x, prepared.lo, prepared.scale, w, s, bias, dtype, 0, v) for w, s, bias in zip(weights, scales, biases)]
+             for v in (wq.MID_TILES[path], wq.TILES[path][0])]
     monkeypatch.setattr(wq, "_segment_plans", {(path, m, rows, 3, k, 0): (wq.MID_TILES[path], 0)})
-    outputs = [torch.empty(m, rows, dtype=torch.bfloat16, device="cuda") for _ in range(3)]
+    monkeypatch.setattr(wq._native.gpu(x), "cus", cus)
+    outputs = [torch.empty(m, rows, dtype=dtype, device="cuda") for _ in range(3)]
+    print(f"mid segments {path} m={m} rows={rows} k={k} cus={cus} {dtype}", flush=True)
     wq.linear_prepared_segments(prepared, weights, scales, biases, outputs)
-    for w, s, bias, y in zip(weights, scales, biases, outputs):
-        want = wq.gemm(prepared.x, prepared.lo, prepared.scale, w, s, bias, torch.bfloat16, 0, wq.MID_TILES[path])
-        assert torch.equal(y, want)
+    torch.cuda.synchronize()
+    for want in wants:
+        assert all(torch.equal(y, w) for y, w in zip(outputs, want))
 
 
 def test_mid_pieces_replay_in_a_graph(wq):

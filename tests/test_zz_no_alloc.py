@@ -33,7 +33,8 @@ def p(t):
     return None if t is None else t.data_ptr()
 
 
-@pytest.mark.parametrize("mode,variant", [("block", 10), ("block", 11), ("block", 15), ("block+g", 12), ("exact+g", 14), ("row", 0), ("exact", 1)])
+@pytest.mark.parametrize("mode,variant", [("block", 10), ("block", 11), ("block", 15), ("block+g", 12), ("exact+g", 14), ("row", 0), ("exact", 1),
+                                          ("row", 16), ("exact", 17), ("block", 18), ("block+g", 19), ("exact+g", 20)])
 def test_noalloc_equals_gemm(wq, mode, variant):
     lib = wq.library()
     stream = torch.cuda.current_stream().cuda_stream
@@ -55,7 +56,9 @@ def test_noalloc_equals_gemm(wq, mode, variant):
 
 
 @pytest.mark.parametrize("mode,variant,shape", [("block", 15, (70, 900, 4096)), ("block", 10, (200, 300, 2048)), ("row", 6, (90, 700, 3072)),
-                                                ("exact", 7, (60, 500, 2048)), ("block", 10, (300, 500, 3072))], ids=str)
+                                                ("exact", 7, (60, 500, 2048)), ("block", 10, (300, 500, 3072)),
+                                                ("row", 16, (90, 700, 8192)), ("exact", 17, (60, 500, 4096)), ("block", 18, (70, 900, 4096)),
+                                                ("block+g", 19, (70, 900, 4096)), ("exact+g", 20, (60, 500, 4096))], ids=str)
 def test_noalloc_split_equals_gemm(wq, mode, variant, shape):
     """With split 1 (the deep split of launches of few tiles: partial planes in the array and a second launch; with 4 CUs
     counted, the split-K tail with its counters in the array, cleared by a kernel): the same bits as wq8_gemm with a

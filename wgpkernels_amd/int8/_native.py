@@ -47,6 +47,7 @@ OPTIONAL = {"wq8_gemm_segments", "wq8_gemm_noalloc", "wq8_quantize_at", "wq8_qua
 TEST_SIGNATURES = {
     "wq8_debug_block_sums": ("i", "ppp" "iii" "i" "p"),
     "wq8_debug_mfma_probe": ("i", "pp" "iii" "p"),
+    "wq8_debug_mid_plan": ("i", "iiiiiii" "p"),
 }
 
 

@@ -94,3 +94,16 @@ WQ8_API int wq8_debug_mfma_probe(const void* operands, int* out, int blocks, int
     else mfma_probe16<<<blocks, 256, 0, stream>>>(static_cast<const v4i*>(operands), out, iters);
     return int(hipGetLastError());
 }
+
+// plan = {tokens and channels of the tile, K pieces} that mid_plan gives a mid variant; segments of seg_rows rows each where
+// that is not 0. Host only.
+WQ8_API int wq8_debug_mid_plan(int m, int n, int k, int variant, int sms, int split, int seg_rows, int* plan) {
+    Variant v;
+    if (!variant_info(variant, v) || v.tile != TILE_MID || m <= 0 || n <= 0 || k <= 0) return -2;
+    GemmArgs g{};
+    g.m = m; g.n = n; g.k = k; g.kblocks = (k + 127) / 128; g.sms = sms; g.seg_rows = seg_rows;
+    const MidPlan p = mid_plan(g, v, split);
+    if (p.shape < 0) return -3;
+    plan[0] = MID_SHAPES[p.shape].bm; plan[1] = MID_SHAPES[p.shape].bn; plan[2] = p.pieces;
+    return 0;
+}
