@@ -58,15 +58,18 @@ int wq8_rotate_groups(const void* x, void* out, int m, int k, int64_t ldx, int d
 
 /* Y (m, n) = epilogue(A (m, k) int8 [, A_lo], B (n, k) int8); variant ids keep the reference's modes: 0, 2, 6 row;
  * 1, 7 exact (a_lo required); 10, 11 block (sa (m, ceil(k/128))); 12, 13 block with weight scales sb (n, ceil(k/128));
- * 14 exact with such weight scales; 15 (no counterpart in the reference) the short block tile with 10's biased fold. k % 16 == 0. Replaces K8:1648; bound at I:79. */
+ * 14 exact with such weight scales. Ids with no counterpart in the reference: 15 the short block tile with 10's biased
+ * fold; 16 row, 17 exact, 18 block (biased fold), 19 block and 20 exact with weight scales sb, on tiles for launches of
+ * about one tile per compute unit. k % 16 == 0. Replaces K8:1648; bound at I:79. */
 int wq8_gemm(const int8_t* a, const int8_t* a_lo, const float* sa, const int8_t* b, const float* sb, const void* bias, const void* residual,
              const void* rscale, void* y, int m, int n, int k, int dtype, int variant, int sms, int split, int* workspace, int* counters,
              wq8_stream_t stream);
 
-/* Workspace bytes {slots, counters} of a wq8_gemm call: slots = the block modes' transposed scales, then with split != 0
- * the split-K partial sums (per split tile, or whole m x n planes per piece for launches of few tiles); counters = one
- * int per tail-split tile (zero on entry, left zero). wq8_gemm returns -2 for a workspace that is not 16-byte aligned.
- * Replaces K8:1506; bound at I:80-81. */
+/* Workspace bytes {slots, counters} of a wq8_gemm call. Variants 0-15: slots = the block scales transposed (sa of the block
+ * modes, sb where it is per k-block), then with split != 0 the split-K partial sums (per split tile, or whole m x n planes
+ * per piece for launches of few tiles); counters = one int per tail-split tile (zero on entry, left zero). Variants 16-20
+ * read the scales as they are: slots = whole m x n planes per K piece with split != 0 (0 bytes for one piece; two planes
+ * a piece for 17), no counters. wq8_gemm returns -2 for a workspace that is not 16-byte aligned. Replaces K8:1506; bound at I:80-81. */
 void wq8_gemm_workspace(int m, int n, int k, int variant, int sms, int split, int64_t* sizes);
 
 /* Untuned variant choice for the row (hilo 0) or exact (hilo 1) mode. Replaces K8:1564; bound at I:82. */
@@ -79,7 +82,8 @@ int wq8_gemm_at(const int8_t* a, const int8_t* a_lo, const float* sa, const int8
                 const long long* counter, long long first, long long step, long long span, long long scale_step, long long in_first,
                 long long in_step, wq8_stream_t stream);
 
-/* 1 to 4 linears of one prepared input in one launch: ys[s] (m, rows) = A @ (bs[s] * sbs[s]).T + biases[s]; rows % 8 == 0.
+/* 1 to 4 linears of one prepared input in one launch: ys[s] (m, rows) = A @ (bs[s] * sbs[s]).T + biases[s]; rows % 8 == 0,
+ * per-channel scales, whole K whatever split says (size the workspace with split 0).
  * Replaces K8:1663; bound at I:88-89 (hasattr-gated). */
 int wq8_gemm_segments(const int8_t* a, const int8_t* a_lo, const float* sa, const int8_t* const* bs, const float* const* sbs,
                       const void* const* biases, void* const* ys, int count, int rows, int m, int k, int dtype, int variant, int sms,

@@ -208,8 +208,9 @@ def rotate_groups(x, group):
 # not use); 11 is the short tile in the reference's fold order.
 TILES = {"row": (0, 6), "exact": (1, 7), "block": (10, 15), "block+g": (12, 13), "exact+g": (14, None)}
 # Per mode: the tiles for launches of about one tile per CU (ids the reference does not use). They were faster than the
-# short tiles at every shape measured (M = 48-2000, K = 1536-13824, N = 1536-13824: by 3-50%), so the timed choice compares
-# them with the long ones; the short tiles run when asked for by id, untimed, and in the path choice (_drawn_runs).
+# short tiles at every shape measured (M = 1-2000, K = 1536-13824, N = 1536-13824: by 3-100%) but four, which were within 1.5%
+# (M = 1-128 row and exact), so the timed choice compares them with the long ones; the short tiles run when asked for by id,
+# untimed, in the path choice (_drawn_runs) and in segments, which have two of the mid tiles only.
 MID_TILES = {"row": 16, "exact": 17, "block": 18, "block+g": 19, "exact+g": 20}
 VARIANT_MODES = {0: "row", 2: "row", 6: "row", 1: "exact", 7: "exact", 10: "block", 11: "block", 12: "block+g", 13: "block+g",
                  14: "exact+g", 15: "block", **{v: mode for mode, v in MID_TILES.items()}}
